@@ -19,7 +19,6 @@ struct dev_tables {
     const uint16_t *cvt16;
     const float *rev16;
     const int16_t *gauss16;
-    const int32_t *gauss16m;   // the Monte adder's LDS image (host_tables::gauss16m, db's dither entries as (-F, 63))
     const uint16_t *exp16;
     const uint16_t *sig16;
     const int32_t *tab32;
@@ -30,6 +29,14 @@ struct dev_tables {
     const uint16_t *lfsr_log;
     const uint16_t *rho16;  // rho16[c] = cvt16 of rev16[c]: a code through F32 and back, as between graph nodes
     const double *lpdb;     // lpvip's db tables (host_tables::lpdb)
+    const int16_t *eb;      // the base adder's table by word distance (eform)
+    const int32_t *em;      // the Monte adder's
+    const int16_t *ebp;     // the same for positive sums
+    const uint16_t *emp;
+    // eight LFSR steps: [0, 256) the draws by the state's low byte, [256, 512)
+    // by its high byte, then 256 uint16: the state eight steps on by its low
+    // byte (its high byte's part is the byte itself)
+    const uint64_t *lfsr8;
 };
 
 __device__ __forceinline__ uint32_t f32_bits(float f) { return __float_as_uint(f); }

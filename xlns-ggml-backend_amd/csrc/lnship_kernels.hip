@@ -273,6 +273,12 @@ __global__ void k_act(const float *__restrict__ x, int64_t x_ld, int64_t x_slice
 
 // |a - b| as one v_sad_u32 (max - min + z, z = 0 held in a register)
 __device__ __forceinline__ uint32_t absdiff(uint32_t a, uint32_t b, uint32_t z) { return max(a, b) - min(a, b) + z; }
+// the same written out, for any z (an address)
+__device__ __forceinline__ uint32_t sad_u32(uint32_t a, uint32_t b, uint32_t z) {
+    uint32_t r;
+    asm("v_sad_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(z));
+    return r;
+}
 __device__ __forceinline__ uint32_t absdiff(uint32_t a, uint32_t b) {
     uint32_t r;
     asm("v_sad_u32 %0, %1, %2, 0" : "=v"(r) : "v"(a), "v"(b));
@@ -362,74 +368,6 @@ struct acc_ls {
 
 template <int MODE>
 struct red16;
-
-template <>
-struct red16<LNSHIP_BASE> {
-    const char *g;   // LDS: (sb, db) int16 pairs per distance d <= esszer + 1
-    using acc_t = acc_ls;
-    __device__ __forceinline__ acc_t start(uint32_t v, uint32_t &) const { return {v & k16_logmask, v & k16_sign}; }
-    __device__ __forceinline__ void add_ls(acc_t &a, uint32_t tl, uint32_t ts, uint32_t &) const {
-        const uint32_t d = absdiff(a.l, tl), mx = max(a.l, tl);
-        const uint32_t usedb = a.s ^ ts;
-        // the sign picks the pair half off the critical path: the address is
-        // then one shift-add of the clamped distance
-        const char *gs = g + (usedb >> 14);
-        const int32_t adj = *reinterpret_cast<const int16_t *>(gs + (min(d, (uint32_t)k16_esszer + 1) << 2));
-        const uint32_t ns = a.l > tl ? a.s : ts;
-        a.l = (uint32_t)min(max((int32_t)mx + adj, 0), (int32_t)k16_logmask);
-        a.s = (d == 0 && usedb) ? 0u : ns;
-    }
-    __device__ __forceinline__ void add(acc_t &a, uint32_t v, uint32_t &st) const { add_ls(a, v & k16_logmask, v & k16_sign, st); }
-    // add() of a positive v to a positive sum (sums of squares, of exps): sb
-    // only, the sign stays +
-    __device__ __forceinline__ void add_pos(acc_t &a, uint32_t v, uint32_t &) const {
-        const uint32_t tl = v & k16_logmask;
-        const uint32_t d = absdiff(a.l, tl), mx = max(a.l, tl);
-        const int32_t adj = *reinterpret_cast<const int16_t *>(g + (min(d, (uint32_t)k16_esszer + 1) << 2));
-        a.l = (uint32_t)min(max((int32_t)mx + adj, 0), (int32_t)k16_logmask);
-    }
-    __device__ __forceinline__ uint32_t finish(const acc_t &a) const { return a.s | a.l; }
-};
-
-template <>
-struct red16<LNSHIP_MONTE> {
-    const int32_t *gm;   // LDS: (sb e, sb m, db e, db m) per distance
-    uint32_t gb;         // gm's LDS byte address
-    using acc_t = acc_ls;
-    __device__ __forceinline__ acc_t start(uint32_t v, uint32_t &) const { return {v & k16_logmask, v & k16_sign}; }
-    // One LFSR step; below the dither range the base table's adjustment, from
-    // it on one ulp toward the smaller operand with probability F(d)/64,
-    // decided by the top 6 bits r of the new state: sb adds (F + r) >> 6,
-    // db (64 - F + ~r) >> 6, here (-F + (63 - r)) >> 6 from the image's
-    // (-F, 63).  The larger log is added scaled by 64 in the same add, so
-    // after the table read only a mask, an add, a shift and the clamp remain.
-    // The sign: the larger operand's (bit 15 of tl - a.l is set iff a.l >
-    // tl), + for exact cancellation (bit 15 of d - 1 is set iff d = 0).
-    __device__ __forceinline__ void add_ls(acc_t &a, uint32_t tl, uint32_t ts, uint32_t &st) const {
-        st = lfsr_step(st);
-        const uint32_t d = absdiff(a.l, tl), mx = max(a.l, tl);
-        const uint32_t usedb = a.s ^ ts;   // 0 or k16_sign
-        // row min(d, end) of 16 bytes, db's pair 8 bytes in
-        const i32x2 em = lds_ld2(lds_at4(min(d, (uint32_t)k16_mc_end), gb + (usedb >> 12)));
-        // the draw r, or 63 - r for db (r xor all ones under the mask 63)
-        const uint32_t x = ((st >> 10) ^ (uint32_t)((int32_t)(usedb << 16) >> 31)) & (uint32_t)em.y;
-        const int32_t sum = (int32_t)(mx << 6) + em.x + (int32_t)x;
-        a.s = bfi(tl - a.l, a.s, ts) & ~(usedb & (d - 1u));
-        a.l = (uint32_t)min(max(sum >> 6, 0), (int32_t)k16_logmask);
-    }
-    __device__ __forceinline__ void add(acc_t &a, uint32_t v, uint32_t &st) const { add_ls(a, v & k16_logmask, v & k16_sign, st); }
-    // add() of a positive v to a positive sum: sb's half of the row, no
-    // sign work (the same draws)
-    __device__ __forceinline__ void add_pos(acc_t &a, uint32_t v, uint32_t &st) const {
-        st = lfsr_step(st);
-        const uint32_t tl = v & k16_logmask;
-        const uint32_t d = absdiff(a.l, tl), mx = max(a.l, tl);
-        const i32x2 em = lds_ld2(lds_at4(min(d, (uint32_t)k16_mc_end), gb));
-        const int32_t sum = (int32_t)(mx << 6) + em.x + (int32_t)((st >> 10) & (uint32_t)em.y);
-        a.l = (uint32_t)min(max(sum >> 6, 0), (int32_t)k16_logmask);
-    }
-    __device__ __forceinline__ uint32_t finish(const acc_t &a) const { return a.s | a.l; }
-};
 
 // xlns32 addition (xlns32_alt), branch-free.  The Gaussian log at distance
 // d has three exclusive cases: sb(d) for equal signs; db(d) from its tables
@@ -795,28 +733,182 @@ __device__ __forceinline__ void stage_copy(int4 *dst, const int4 *__restrict__ s
     }
 }
 
+// ---- base and Monte sums as one word ------------------------------------------
+// The base and Monte adders on a value held in one word, E = (log + k16_one)
+// 2^sh + (u if negative), u = 2^sh / 4: the signed maximum of two words is the
+// larger operand with its sign (on equal logs the negative one), and the
+// distance of two words is v = d 2^sh for equal signs, d 2^sh +- u for opposite
+// ones.  v itself is the byte offset of the adjustment: the table has four
+// slots per distance, sb(d) in slot 0, db(d) in the slots above and below, so a
+// step is the maximum, the distance, its cap, the read and one shift-add, with
+// no work for the signs: 6 instructions besides the product, against 16 with
+// the log and the sign in separate words.
+//
+// The steps clamp nothing: the fast form of a step is exact when the larger
+// operand's log is at least `far` (the distance from which an addend adds
+// nothing) and at most k16_logmask.  Below that, the log of a product may be
+// less than 0 (its clamp makes it 0), which then lies far enough from the sum
+// either way; exact cancellation leaves a negative word, which every later
+// term exceeds from beyond `far`.  The chains run in blocks: a block records
+// the least and the largest M of its steps, and one that leaves the range is
+// run again by the exact form (xstep), which clamps.
+//
+// Measured on MI355X against the clamping adder with log and sign apart: a
+// single chain's step 51 -> 38 ns (base) and 65 -> 49 ns (Monte); the product
+// K 2048, M 8192, N 512 1913 -> 4220 GMAC/s (base), 1341 -> 2569 (Monte).
+//
+// POS: sums of positive terms only (squares, exps): E = 2 log, one 16-bit
+// entry per distance, no signs; the sums only grow, so a block is in range when
+// it starts at lo or above and ends at hi or below.
+template <int MODE, bool POS = false>
+struct eform {
+    static constexpr bool monte = MODE == LNSHIP_MONTE;
+    static constexpr int sh = POS ? 1 : monte ? 4 : 3;   // slots of 4 (Monte) or 2 bytes
+    static constexpr uint32_t u = POS ? 0u : 1u << (sh - 2);
+    static constexpr int far = monte ? k16_mc_end : k16_esszer + 1;   // table entry `far` is 0
+    static constexpr uint32_t cap = (uint32_t)far << sh;
+    static constexpr int bytes = ((int)cap + 4 + 15) & ~15;           // of the table
+    static constexpr uint32_t bias = POS ? 0u : k16_one;              // (a product's log is that of its word less k16_one)
+    static constexpr int32_t lo = (int32_t)((bias + far) << sh);
+    static constexpr int32_t hi = (int32_t)(((bias + k16_logmask) << sh) | u);
+    static constexpr int32_t zero = (int32_t)(bias << sh);
+};
+// the word of an xlns16 code
+template <int MODE>
+__device__ __forceinline__ int32_t e_of(uint32_t c) {
+    using E = eform<MODE>;
+    return (int32_t)((((c & k16_logmask) + k16_one) << E::sh) | (((c >> 15) & 1u) << (E::sh - 2)));
+}
+// The words of two products whose codes' halves are in w and x, in two parts:
+// the log fields added (no carry crosses the halves) and the signs xor'ed and
+// moved to u's place in each half; then the two words
+template <int MODE>
+__device__ __forceinline__ void e_pair(uint32_t w, uint32_t x, uint32_t k_lm, uint32_t k_su, uint32_t &lm, uint32_t &sg) {
+    lm = (w & k_lm) + (x & k_lm);
+    sg = ((w ^ x) >> (15 - (eform<MODE>::sh - 2))) & k_su;
+    asm("" : "+v"(lm), "+v"(sg));   // (opaque: the inserts below stay one instruction each)
+}
+template <int MODE>
+__device__ __forceinline__ void e_words(uint32_t lm, uint32_t sg, uint32_t k_em, int32_t (&t)[2]) {
+    t[0] = (int32_t)bfi(k_em, lm << eform<MODE>::sh, sg);
+    t[1] = (int32_t)bfi(k_em, lm >> (16 - eform<MODE>::sh), sg >> 16);
+}
+struct e_masks {
+    uint32_t lm, em, su;
+};
+template <int MODE>
+__device__ __forceinline__ e_masks e_mask_regs() {
+    using E = eform<MODE>;
+    e_masks k{0x7fff7fffu, 0xffffu << E::sh, E::u * 0x10001u};
+    asm("" : "+v"(k.lm), "+v"(k.em), "+v"(k.su));
+    return k;
+}
+typedef const int16_t __attribute__((address_space(3))) *lds_i16_t;
+typedef const uint16_t __attribute__((address_space(3))) *lds_u16_t;
+template <int MODE, bool POS = false>
+struct red_e {
+    using E = eform<MODE, POS>;
+    uint32_t tb, cap;   // LDS byte addresses of the table and of its last entry
+    uint32_t scale;     // 2^sh in a register the compiler cannot see into
+    // non-null: the table in global memory, for launches whose rows leave no
+    // room for it in LDS (tb is 0); only exact steps run then
+    const char *g;
+    // the address of the entry for words x and y: their distance, the table's
+    // base added by the same instruction, capped
+    __device__ __forceinline__ uint32_t at(int32_t x, int32_t y) const {
+        return min(sad_u32((uint32_t)x, (uint32_t)y, tb), cap);
+    }
+    __device__ __forceinline__ int32_t entry(uint32_t va) const {
+        if constexpr (E::monte && !POS) return lds_ld(va);
+        else if constexpr (E::monte) return *(lds_u16_t)(uintptr_t)va;
+        else return *(lds_i16_t)(uintptr_t)va;
+    }
+    __device__ __forceinline__ int32_t entry_any(uint32_t va) const {
+        if (__builtin_expect(g == nullptr, 1)) return entry(va);
+        if constexpr (E::monte && !POS) return *reinterpret_cast<const int32_t *>(g + va);
+        else if constexpr (E::monte) return *reinterpret_cast<const uint16_t *>(g + va);
+        else return *reinterpret_cast<const int16_t *>(g + va);
+    }
+    // the sum: the larger word M and the adjustment of entry en at address va;
+    // r: Monte's draw, the top 6 bits of the LFSR state.  Monte's entries are
+    // (64 adj or F) for equal signs, to which r is added, and (64 adj + 64 or
+    // 64 - F) for opposite ones, to which ~r is added: the carry out of the
+    // low 6 bits is the draw's ulp, and outside the dither range (F = 0)
+    // there is none.
+    static __device__ __forceinline__ uint32_t draw(uint32_t va, uint32_t r) {
+        if constexpr (POS) return r;
+        else return r ^ (uint32_t)__builtin_amdgcn_sbfe((int32_t)va, E::sh - 2, 1);
+    }
+    static __device__ __forceinline__ int32_t sum(int32_t M, int32_t en, uint32_t dr) {
+        if constexpr (E::monte) return (int32_t)((uint32_t)((int32_t)(dr + (uint32_t)en) >> 6) << E::sh) + M;
+        else return (int32_t)((uint32_t)en << E::sh) + M;
+    }
+    // a <- a (+) t, exact for lo <= M <= hi
+    __device__ __forceinline__ void step(int32_t &a, int32_t t, uint32_t r, int32_t &M) const {
+        const uint32_t va = at(a, t);
+        M = max(a, t);
+        a = sum(M, entry(va), draw(va, r));
+    }
+    // The same for a single chain, where every instruction of the wave is on
+    // the chain's clock: the read goes out first, then the maximum and
+    // shadow()'s work (the next products) run in its round trip.
+    template <class F>
+    __device__ __forceinline__ int32_t step1(int32_t &a, int32_t t, uint32_t r, F &&shadow) const {
+        uint32_t va;
+        asm("v_sad_u32 %0, %1, %2, %3\n\tv_min_u32 %0, %0, %4" : "=&v"(va) : "v"(a), "v"(t), "v"(tb), "v"(cap));
+        const int32_t en = entry(va);
+        __builtin_amdgcn_sched_barrier(0);
+        const int32_t M = max(a, t);
+        const uint32_t dr = E::monte ? draw(va, r) : 0u;
+        shadow();
+        asm volatile("" ::"v"(M), "v"(dr));
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (E::monte) a = __mul24((int32_t)(dr + (uint32_t)en) >> 6, (int32_t)scale) + M;   // (one v_mad: as a shift the compiler makes two)
+        else a = sum(M, en, dr);
+        return M;
+    }
+    // a word as the reference's clamps leave it: the log within its field,
+    // the sign kept
+    static __device__ __forceinline__ int32_t clamped(int32_t e) {
+        return (int32_t)bfi(E::u, (uint32_t)e, (uint32_t)min(max(e, E::zero), E::hi));
+    }
+    // a sum after fast steps: only exact cancellation (+0) leaves it below zero
+    static __device__ __forceinline__ int32_t settled(int32_t e) { return e < E::zero ? E::zero : clamped(e); }
+    // the step for any operands; a comes and goes clamped
+    __device__ __forceinline__ void xstep(int32_t &a, int32_t t, uint32_t r, int32_t &M) const {
+        t = clamped(t);
+        M = max(a, t);
+        const uint32_t va = at(a, t);
+        const int32_t x = sum(M, entry_any(va), draw(va, r));
+        a = !POS && va == tb + E::u ? E::zero : clamped(x);   // exact cancellation: +0
+    }
+    // the xlns16 code of a sum
+    static __device__ __forceinline__ uint32_t finish(int32_t e) {
+        const uint32_t c = (uint32_t)settled(e);
+        if constexpr (POS) return c >> E::sh;
+        else return ((c >> E::sh) - k16_one) | ((c & E::u) << (15 - (E::sh - 2)));
+    }
+};
+template <int MODE, bool POS>
+__device__ __forceinline__ const char *e_image(const dev_tables &T) {
+    if constexpr (MODE == LNSHIP_MONTE) return POS ? (const char *)T.emp : (const char *)T.em;
+    else return POS ? (const char *)T.ebp : (const char *)T.eb;
+}
+// the table image into LDS, or (in_lds false) left in global memory
+template <int MODE, bool POS = false>
+__device__ __forceinline__ red_e<MODE, POS> stage_e(const dev_tables &T, char *lds, bool in_lds = true) {
+    using E = eform<MODE, POS>;
+    const char *img = e_image<MODE, POS>(T);
+    if (in_lds) stage_copy<8>(reinterpret_cast<int4 *>(lds), reinterpret_cast<const int4 *>(img), E::bytes / 16);
+    const uint32_t tb = in_lds ? lds_addr(lds) : 0u;
+    red_e<MODE, POS> R{tb, tb + E::cap, 1u << E::sh, in_lds ? nullptr : img};
+    asm("" : "+v"(R.tb), "+v"(R.cap), "+v"(R.scale));   // in registers (short encodings)
+    return R;
+}
+
 template <int MODE>
 __device__ __forceinline__ red16<MODE> stage_tables(const dev_tables &T, char *lds);
 
-template <>
-__device__ __forceinline__ red16<LNSHIP_BASE> stage_tables<LNSHIP_BASE>(const dev_tables &T, char *lds) {
-    int16_t *g = reinterpret_cast<int16_t *>(lds);
-    for (int i = threadIdx.x; i < k16_gauss_n; i += blockDim.x) {
-        g[2 * i] = T.gauss16[i];
-        g[2 * i + 1] = i == 0 ? (int16_t)-32768 : T.gauss16[k16_gauss_n + i];
-    }
-    return red16<LNSHIP_BASE>{lds};
-}
-template <>
-__device__ __forceinline__ red16<LNSHIP_MONTE> stage_tables<LNSHIP_MONTE>(const dev_tables &T, char *lds) {
-    int32_t *g = reinterpret_cast<int32_t *>(lds);
-    stage_copy<8>(reinterpret_cast<int4 *>(g), reinterpret_cast<const int4 *>(T.gauss16m), k16_mc_n);
-    // db at distance 0: an adjustment that clamps the log to 0 (exact
-    // cancellation; the sign is cleared by the caller).  Thread 0 copied
-    // that entry itself, so its own later store wins.
-    if (threadIdx.x == 0) g[2] = -(1 << 30);
-    return red16<LNSHIP_MONTE>{g, lds_addr(g)};
-}
 // img: one of the two images built at init (lds32_image): the multi-chain
 // step's, or the single-chain step's
 __device__ __forceinline__ red16<LNSHIP_SUM32> stage_x32(const int32_t *img, char *lds) {
@@ -882,6 +974,8 @@ __device__ __forceinline__ red16<MODE> stage_for(const dev_tables &T, char *lds)
     else return stage_tables<MODE>(T, lds);
 }
 
+// (base and Monte: not their tables' size, which each kernel states, but what
+// bounds the rows that the entry points accept, lnship_max_row)
 template <int MODE>
 constexpr int lds_tables_bytes() {
     return MODE == LNSHIP_BASE ? 2 * k16_gauss_n * 2 :
@@ -892,17 +986,17 @@ constexpr int lds_tables_bytes() {
 // chains add only positive values (squares, exps), over the positive-sum
 // adder's pair image; the other modes stage their adder's tables.
 template <int MODE>
+constexpr bool is_e = MODE == LNSHIP_BASE || MODE == LNSHIP_MONTE;   // the one-word adders
+template <int MODE>
 constexpr int row_tables_bytes() {
-    return MODE == LNSHIP_SUM32 ? k_lds_pos32 : lds_tables_bytes<MODE>();
+    if constexpr (is_e<MODE>) return eform<MODE, true>::bytes;
+    else return MODE == LNSHIP_SUM32 ? k_lds_pos32 : lds_tables_bytes<MODE>();
 }
 template <int MODE>
-__device__ __forceinline__ red16<MODE> stage_rows(const dev_tables &T, char *lds, pos_tab &P) {
-    if constexpr (MODE == LNSHIP_SUM32) {
-        P = stage_pos32(T, lds);
-        return red16<MODE>{};
-    } else {
-        return stage_tables<MODE>(T, lds);
-    }
+__device__ __forceinline__ auto stage_rows(const dev_tables &T, char *lds) {
+    if constexpr (MODE == LNSHIP_SUM32) return stage_pos32(T, lds);
+    else if constexpr (is_e<MODE>) return stage_e<MODE, true>(T, lds);
+    else return stage_tables<MODE>(T, lds);
 }
 
 // ---- MUL_MAT ------------------------------------------------------------------
@@ -951,6 +1045,9 @@ struct mm_args16 {
     // Monte start, monte_start(rms_seed, state, rms_offset)
     uint32_t rms_seed;
     uint64_t rms_offset;
+    // set by the launcher (base and Monte, one chain per lane): the rows leave
+    // no room for the adder's table in LDS
+    bool no_tab;
     // set by the launcher: the grid is 2^xcd_sh times wider than the work;
     // workgroup x works (as block x >> xcd_sh) iff x is a multiple of 2^xcd_sh
     uint32_t xcd_sh;
@@ -987,6 +1084,14 @@ __device__ __forceinline__ uint32_t monte_start(const dev_tables &T, uint32_t se
 
 template <int MODE>
 constexpr int mm_xl_offset() { return (lds_tables_bytes<MODE>() + 15) & ~15; }
+// k_mm16's own tables: the one-word adders' for base and Monte, with the LFSR
+// tables when a lane runs several Monte chains
+constexpr int k_lfsr8_bytes = 2 * 256 * 8 + 256 * 2;
+template <int MODE>
+constexpr int mm16_tab_bytes() {
+    if constexpr (is_e<MODE>) return eform<MODE>::bytes + (MODE == LNSHIP_MONTE ? k_lfsr8_bytes : 0);
+    else return mm_xl_offset<MODE>();
+}
 // LDS padding past the activation rows (a block's prefetch reads up to that
 // far past the last column)
 constexpr int k_xl_pad = 8 * 16;
@@ -1288,6 +1393,394 @@ __device__ __forceinline__ void mm16_chains(const mm_args16 &a, const dev_tables
     for (int j = 0; j < NC; j++) res[j] = R.finish(acc[j]) & 0xffffu;
 }
 
+// (defined with the other sequential row sums below)
+template <int MODE, bool POS>
+__device__ __forceinline__ uint32_t chain_e_pos(const red_e<MODE, POS> &R, uint32_t a, const uint16_t *row, int i0,
+                                                int n, uint32_t st);
+template <class RED, bool POS = false>
+__device__ __forceinline__ void chain16(const RED &R, typename RED::acc_t &acc, const uint16_t *row, int i0, int n,
+                                        uint32_t &st);
+
+// Eight LFSR steps at once: the draws r of states 1 .. 8 on from s, a byte
+// each, and the state eight on, from three LDS reads (the LFSR is linear: its
+// low and high bytes' parts are xor'ed)
+struct lfsr8_tab {
+    uint32_t lo, t8;   // LDS byte addresses
+};
+__device__ __forceinline__ lfsr8_tab stage_lfsr8(const dev_tables &T, char *lds) {
+    stage_copy<2>(reinterpret_cast<int4 *>(lds), reinterpret_cast<const int4 *>(T.lfsr8), k_lfsr8_bytes / 16);
+    return {lds_addr(lds), lds_addr(lds) + 4096u};
+}
+__device__ __forceinline__ i32x2 lfsr_draws8(const lfsr8_tab &L, uint32_t &s) {
+    const uint32_t b = s & 255u, h = s >> 8;
+    const i32x2 x = lds_ld2(L.lo + (b << 3)) ^ lds_ld2(L.lo + 2048u + (h << 3));
+    s = h ^ (uint32_t) * (const uint16_t __attribute__((address_space(3))) *)(uintptr_t)(L.t8 + (b << 1));
+    return x;
+}
+
+// mm16_chains for base and Monte, over the one-word adders.  X32: the
+// activation rows are words in LDS ((log << sh) | u if negative), NC > 1; else
+// codes, in LDS (XL) or in scratch, and a column's products are formed two at a
+// time in 16-bit halves.  Several chains per lane are bound by LDS reads and
+// instruction issue: a weight's word is formed once for its NC products, each
+// of which is then one shift-add and one mask, and Monte's draws come eight at a time
+// from tables.
+template <int MODE, int NC, int PF, bool XL, bool X32>
+__device__ __forceinline__ void mme_chains(const mm_args16 &a, const dev_tables &T, const red_e<MODE> &R,
+                                           const lfsr8_tab &L8, const void *xl, int64_t m, int64_t z, int64_t zw,
+                                           int64_t zx, int64_t n0, int nc, uint32_t (&res)[NC]) {
+    using E = eform<MODE>;
+    constexpr bool monte = E::monte;
+    const int kp = (int)a.kp, K = (int)a.K;
+    const uint16_t *ws = a.w + zw * a.w_slice + m * 8;
+    const uint16_t *xs = a.x + (zx * a.N + n0) * a.kp;
+    const int64_t wstride = a.w_mstride * 8;
+    const int full = K >> 3, tail = K & 7, last = (kp >> 3) - 1;
+    int32_t acc[NC];
+    uint32_t st[NC];
+#pragma unroll
+    for (int j = 0; j < NC; j++) {
+        acc[j] = E::zero;
+        st[j] = 0;
+        // one draw before the first: step 0 of the chain, which starts the
+        // sum, takes a draw that nothing reads
+        if (monte && j < nc) {
+            const uint64_t out = ((uint64_t)z * (uint64_t)a.M + (uint64_t)m) * (uint64_t)a.N + (uint64_t)(n0 + j);
+            st[j] = lfsr_jump(T, monte_start(T, a.seed, a.state, a.offset), out * (uint64_t)(a.K - 1) + 65534u);
+        }
+    }
+    const e_masks km = e_mask_regs<MODE>();
+    auto load_w = [&](int g) { return *reinterpret_cast<const uint4 *>(ws + (int64_t)min(g, last) * wstride); };
+    struct grp_x {
+        uint4 q[X32 ? 2 : 1];
+    };
+    // a column's activations of group g (the offset through a vector
+    // register, as in mm16_chains)
+    auto load_x = [&](int j, int g) {
+        grp_x r;
+        if constexpr (X32) {
+            int32_t off = (j * kp + min(g, last) * 8) * 4;
+            asm("" : "+v"(off));
+            const uint4 *p = reinterpret_cast<const uint4 *>(static_cast<const char *>(xl) + off);
+            r.q[0] = p[0];
+            r.q[1] = p[1];
+        } else {
+            int64_t off = (int64_t)(XL || j < nc ? j : 0) * kp + (int64_t)min(g, last) * 8;
+            asm("" : "+v"(off));
+            r.q[0] = *reinterpret_cast<const uint4 *>((XL ? static_cast<const uint16_t *>(xl) : xs) + off);
+        }
+        return r;
+    };
+    // steps [u0, u1) of a group; FAST: the fast form, else the exact one;
+    // start: step 0 starts the sums.  mn, mx: the least and largest M.
+    int32_t mn = E::hi, mx = E::lo;
+    auto group = [&](auto fast_tag, const uint4 &wq, const grp_x (&xq)[NC], int u0, int u1, bool start)
+                     __attribute__((always_inline)) {
+        constexpr bool FAST = decltype(fast_tag)::value;
+        const uint32_t ww[4] = {wq.x, wq.y, wq.z, wq.w};
+        i32x2 dr[NC];
+        if constexpr (monte)
+#pragma unroll
+            for (int j = 0; j < NC; j++) dr[j] = lfsr_draws8(L8, st[j]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (2 * i >= u1 || 2 * i + 1 < u0) continue;
+            int32_t t[NC][2];
+            if constexpr (X32) {
+                // the weights' words over u: a code rotated by its sign
+                const uint32_t w0 = (__builtin_amdgcn_ubfe(ww[i], 0, 15) << 2) | __builtin_amdgcn_ubfe(ww[i], 15, 1);
+                const uint32_t w1 = (__builtin_amdgcn_ubfe(ww[i], 16, 15) << 2) | (ww[i] >> 31);
+#pragma unroll
+                for (int j = 0; j < NC; j++) {
+                    const uint4 &q = xq[j].q[i >> 1];
+                    const uint32_t x0 = (i & 1) ? q.z : q.x, x1 = (i & 1) ? q.w : q.y;
+                    // (two negative factors: the sum of their signs is 2 u)
+                    t[j][0] = (int32_t)(((w0 << (E::sh - 2)) + x0) & ~(2u * E::u));
+                    t[j][1] = (int32_t)(((w1 << (E::sh - 2)) + x1) & ~(2u * E::u));
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < NC; j++) {
+                    const uint4 &q = xq[j].q[0];
+                    uint32_t lm, sg;
+                    e_pair<MODE>(ww[i], i == 0 ? q.x : i == 1 ? q.y : i == 2 ? q.z : q.w, km.lm, km.su, lm, sg);
+                    e_words<MODE>(lm, sg, km.em, t[j]);
+                }
+            }
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int u = 2 * i + h;
+                if (u < u0 || u >= u1) continue;
+                int32_t M[NC];
+#pragma unroll
+                for (int j = 0; j < NC; j++) {
+                    uint32_t r = 0;
+                    if constexpr (monte) r = __builtin_amdgcn_ubfe((uint32_t)(u < 4 ? dr[j].x : dr[j].y), 8 * (u & 3), 8);
+                    if (u == 0 && start) {
+                        acc[j] = red_e<MODE>::clamped(t[j][h]);
+                        M[j] = E::hi;
+                    } else if constexpr (FAST) {
+                        R.step(acc[j], t[j][h], r, M[j]);
+                    } else {
+                        R.xstep(acc[j], t[j][h], r, M[j]);
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < NC; j++) {
+                    mn = min(mn, M[j]);
+                    mx = max(mx, M[j]);
+                }
+            }
+        }
+    };
+    // Group 0 (which starts the sums), then blocks of PF groups, then the
+    // tail: blocks run in the fast form, and again in the exact one when a
+    // step left its range; the next block then starts exact, until one stays
+    // in range.  Group 0 and the tail run exact (one copy of each form's code).
+    // The next block's weights are loaded before a block runs.
+    bool exact = false;   // wave-uniform
+    const int groups = full + (tail > 0);
+    uint4 wa[PF], wb[PF];
+    mm16_wblock<PF>(a, m, zw, 1, wa);
+    for (int g = 0, g1 = 1; g < groups; g = g1, g1 = min(g + PF, g < full ? full : groups)) {
+        const bool body = g > 0 && g < full;
+        mn = E::hi;
+        mx = E::lo;
+        bool redo = true;
+        if (body) {
+            mm16_wblock<PF>(a, m, zw, g + PF, wb);
+            if (!exact) {
+                int32_t a0[NC];
+                uint32_t s0[NC];
+#pragma unroll
+                for (int j = 0; j < NC; j++) {
+                    a0[j] = acc[j];
+                    s0[j] = st[j];
+                }
+#pragma unroll
+                for (int p = 0; p < PF; p++)
+                    if (g + p < full) {
+                        grp_x xq[NC];
+#pragma unroll
+                        for (int j = 0; j < NC; j++) xq[j] = load_x(j, g + p);
+                        group(std::true_type{}, wa[p], xq, 0, 8, false);
+                    }
+                redo = __any(mn < E::lo || mx > E::hi) != 0;
+                if (redo) {
+#pragma unroll
+                    for (int j = 0; j < NC; j++) {
+                        acc[j] = a0[j];
+                        st[j] = s0[j];
+                    }
+                    mn = E::hi;
+                    mx = E::lo;
+                }
+            }
+#pragma unroll
+            for (int p = 0; p < PF; p++) wa[p] = wb[p];
+        }
+        if (redo) {
+#pragma unroll
+            for (int j = 0; j < NC; j++) acc[j] = red_e<MODE>::settled(acc[j]);
+#pragma unroll 1
+            for (int q = g; q < g1; q++) {
+                grp_x xq[NC];
+#pragma unroll
+                for (int j = 0; j < NC; j++) xq[j] = load_x(j, q);
+                group(std::false_type{}, load_w(q), xq, 0, q < full ? 8 : tail, q == 0);
+            }
+            exact = __any(mn < E::lo || mx > E::hi) != 0;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NC; j++) res[j] = red_e<MODE>::finish(acc[j]) & 0xffffu;
+}
+
+// Terms k0 <= k < k1 (k0 < k1) of one chain, added to the sum word acc in order
+// (term 0 starts it): one chain per lane, bound by its dependent path
+// (distance, cap, LDS read, sum).  Each product is formed in the round trips of
+// the two steps before it, two at a time, and the steps are kept in order.
+// Groups of eight terms: the first one's weights in w0, those of the PF after
+// it in wa; block(w, g) loads groups g .. g + PF - 1 (past the last: the last
+// again), load_w(g) and load_x(g) a group's weights and activations.  st:
+// Monte's LFSR state one draw before term 8 (k0 / 8)'s.
+template <int MODE, int PF, class B, class W, class X>
+__device__ __forceinline__ void chain_e(const red_e<MODE> &R, const lfsr8_tab &L8, int32_t &acc, uint32_t st, int k0,
+                                        int k1, const uint4 &w0, uint4 (&wa)[PF], B &&block, W &&load_w, X &&load_x) {
+    using E = eform<MODE>;
+    const int gf = k0 >> 3, full = k1 >> 3, tail = k1 & 7, groups = full + (tail > 0);
+    const e_masks km = e_mask_regs<MODE>();
+    int32_t mn = E::hi, mx = E::lo;   // the least and largest M
+    auto pair = [&](uint32_t w, uint32_t x, int32_t (&t)[2]) {
+        uint32_t lm, sg;
+        e_pair<MODE>(w, x, km.lm, km.su, lm, sg);
+        e_words<MODE>(lm, sg, km.em, t);
+    };
+    // Monte's draws of a group, a byte each, and those of the next one, whose
+    // table reads are in flight meanwhile
+    i32x2 dr{0, 0}, drn{0, 0};
+    auto draw_of = [&](int u) { return E::monte ? __builtin_amdgcn_ubfe((uint32_t)(u < 4 ? dr.x : dr.y), 8 * (u & 3), 8) : 0u; };
+    auto draws = [&](bool fast) __attribute__((always_inline)) {
+        if constexpr (E::monte) {
+            if (!fast && R.g) {   // no tables in LDS: step by step
+                uint32_t d[2] = {0, 0};
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    st = lfsr_step(st);
+                    d[u >> 2] |= (st >> 10) << (8 * (u & 3));
+                }
+                drn = i32x2{(int32_t)d[0], (int32_t)d[1]};
+            } else {
+                drn = lfsr_draws8(L8, st);
+            }
+        }
+    };
+    // The eight steps of a group, its terms 0 and 1 in t0, t1; wn, xn: the
+    // first words of the next group, whose terms 0 and 1 it leaves there.  A
+    // pair of products is formed in two parts, in the round trips of the two
+    // steps before it, and the M of two steps recorded in that of a third.
+    int32_t t0 = 0, t1 = 0, Ma = E::hi, Mb = E::hi;
+    auto note = [&] {
+        asm("v_min3_i32 %0, %0, %1, %2" : "+v"(mn) : "v"(Ma), "v"(Mb));
+        asm("v_max3_i32 %0, %0, %1, %2" : "+v"(mx) : "v"(Ma), "v"(Mb));
+    };
+    auto fast8 = [&](const uint4 &wq, const uint4 &xq, uint32_t wn, uint32_t xn, int u0) __attribute__((always_inline)) {
+        const uint32_t ww[5] = {wq.x, wq.y, wq.z, wq.w, wn}, xx[5] = {xq.x, xq.y, xq.z, xq.w, xn};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            int32_t tn[2], M0 = E::hi;
+            uint32_t lm = 0, sg = 0;
+            auto even = [&] {
+                e_pair<MODE>(ww[i + 1], xx[i + 1], km.lm, km.su, lm, sg);
+                note();
+                asm volatile("" ::"v"(mn), "v"(mx));
+            };
+            if (2 * i >= u0) M0 = R.step1(acc, t0, draw_of(2 * i), even);
+            else even();
+            if (i == 0) draws(true);
+            Mb = R.step1(acc, t1, draw_of(2 * i + 1), [&] {
+                e_words<MODE>(lm, sg, km.em, tn);
+                asm volatile("" ::"v"(tn[0]), "v"(tn[1]));
+            });
+            Ma = M0;
+            t0 = tn[0];
+            t1 = tn[1];
+        }
+        dr = drn;
+    };
+    // steps [u0, u1) of a group in the exact form; start: step 0 starts the sum
+    auto exact8 = [&](const uint4 &wq, const uint4 &xq, int u0, int u1, bool start) __attribute__((always_inline)) {
+        const uint32_t ww[4] = {wq.x, wq.y, wq.z, wq.w}, xx[4] = {xq.x, xq.y, xq.z, xq.w};
+        draws(false);
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            if (u < u0 || u >= u1) continue;
+            int32_t t[2], M = E::hi;
+            pair(ww[u >> 1], xx[u >> 1], t);
+            if (u == 0 && start) acc = red_e<MODE>::clamped(t[0]);
+            else R.xstep(acc, t[u & 1], draw_of(u), M);
+            mn = min(mn, M);
+            mx = max(mx, M);
+        }
+        dr = drn;
+    };
+    draws(false);
+    dr = drn;
+    // as mme_chains: the first group, blocks of PF groups, the tail; a group
+    // or block that left the fast form's range runs again exactly, and so
+    // does the next block, until one stays in range.  The tail, and a first
+    // group that is not a whole one from term 0, run exactly.
+    bool exact = R.g != nullptr;
+    uint4 wb[PF];
+    for (int g = gf, g1 = gf + 1; g < groups; g = g1, g1 = min(g + PF, g < full ? full : groups)) {
+        mn = E::hi;
+        mx = E::lo;
+        bool redo = true;
+        if (g < full && (g > gf || k0 == 0)) {
+            const int32_t a0 = acc;
+            const uint32_t s0 = st;
+            const i32x2 d0 = dr;
+            if (g > gf) block(wb, g + PF);
+            if (!exact) {
+                int32_t t[2];
+                Ma = Mb = E::hi;
+                if (g == gf) {
+                    const uint4 x0 = load_x(gf);
+                    pair(w0.x, x0.x, t);
+                    acc = red_e<MODE>::clamped(t[0]);
+                    t1 = t[1];
+                    fast8(w0, x0, w0.x, x0.x, 1);
+                } else {
+                    uint4 x[PF];
+#pragma unroll
+                    for (int p = 0; p < PF; p++) x[p] = load_x(g + p);
+                    pair(wa[0].x, x[0].x, t);
+                    t0 = t[0];
+                    t1 = t[1];
+#pragma unroll
+                    for (int p = 0; p < PF; p++)
+                        if (g + p < full)
+                            fast8(wa[p], x[p], wa[p + 1 < PF ? p + 1 : p].x, x[p + 1 < PF ? p + 1 : p].x, 0);
+                }
+                note();
+                redo = __any(mn < E::lo || mx > E::hi) != 0;
+                if (redo) {
+                    acc = a0;
+                    st = s0;
+                    dr = d0;
+                    mn = E::hi;
+                    mx = E::lo;
+                }
+            }
+            if (g > gf)
+#pragma unroll
+                for (int p = 0; p < PF; p++) wa[p] = wb[p];
+        }
+        if (redo) {
+            acc = red_e<MODE>::settled(acc);
+#pragma unroll 1
+            for (int q = g; q < g1; q++)
+                exact8(load_w(q), load_x(q), q == gf ? k0 & 7 : 0, q < full ? 8 : tail, q == 0);
+            exact = R.g != nullptr || (g > gf && __any(mn < E::lo || mx > E::hi) != 0);
+        }
+    }
+}
+
+// mme_chains for one chain per lane; head: its first weights
+template <int MODE, int PF, bool XL, bool HEAD>
+__device__ __forceinline__ uint32_t mme_chain1(const mm_args16 &a, const dev_tables &T, const red_e<MODE> &R,
+                                               const lfsr8_tab &L8, const uint16_t *xl, int64_t m, int64_t z,
+                                               int64_t zw, int64_t zx, int64_t n0, const mm_head<PF> &head) {
+    const uint16_t *ws = a.w + zw * a.w_slice + m * 8;
+    const uint16_t *xs = XL ? xl : a.x + (zx * a.N + n0) * a.kp;
+    const int64_t wstride = a.w_mstride * 8;
+    const int last = (int)(a.kp >> 3) - 1;
+    uint32_t st = 0;
+    // one draw before the first: step 0, which starts the sum, takes a draw
+    // that nothing reads
+    if constexpr (MODE == LNSHIP_MONTE) {
+        const uint64_t out = ((uint64_t)z * (uint64_t)a.M + (uint64_t)m) * (uint64_t)a.N + (uint64_t)n0;
+        st = lfsr_jump(T, monte_start(T, a.seed, a.state, a.offset), out * (uint64_t)(a.K - 1) + 65534u);
+    }
+    auto load_w = [&](int g) { return *reinterpret_cast<const uint4 *>(ws + (int64_t)min(g, last) * wstride); };
+    auto load_x = [&](int g) {   // (the offset through a vector register, as in mm16_chains)
+        int32_t off = min(g, last) * 8;
+        asm("" : "+v"(off));
+        return *reinterpret_cast<const uint4 *>(xs + off);
+    };
+    uint4 wa[PF];
+    if constexpr (HEAD) {
+#pragma unroll
+        for (int p = 0; p < PF; p++) wa[p] = head.w[p];
+    } else {
+        mm16_wblock<PF>(a, m, zw, 1, wa);
+    }
+    int32_t acc = eform<MODE>::zero;
+    chain_e<MODE, PF>(R, L8, acc, st, 0, (int)a.K, HEAD ? head.w0 : load_w(0), wa,
+                      [&](uint4 (&w)[PF], int g) { mm16_wblock<PF>(a, m, zw, g, w); }, load_w, load_x);
+    return red_e<MODE>::finish(acc) & 0xffffu;
+}
+
 // W < 64: W rows per wave (single-chain GEMVs, bound by the dependent
 // latency of their chains).  sum32: the wave's other lanes only stage the
 // tables and the activations (a VALU instruction with only the first 16
@@ -1296,8 +1789,13 @@ __device__ __forceinline__ void mm16_chains(const mm_args16 &a, const dev_tables
 // steps branch (lpvip's FP64 Gaussian log, the sign cases) and, measured,
 // run slower with part of the wave inactive (lpvip K 1536: 420 us with 16
 // lanes, 334 us with the same 16 chains on all 64, 313 us with 4 chains)
-template <int MODE, int NC, int PF, bool XL, int CG, int W = 64>
-__global__ __launch_bounds__(k_block * CG) void k_mm16(mm_args16 a, dev_tables T) {
+// X32 (base and Monte, several columns): the activation rows are staged as the
+// one-word adders' words, 4 bytes each, where they fit LDS; RG groups of
+// k_block rows then share them, so that long rows leave room for enough waves
+template <int MODE, int NC, int PF, bool XL, int CG, int W = 64, bool X32 = false, int RG = 1>
+__global__ __launch_bounds__(k_block *CG *RG) void k_mm16(mm_args16 a, dev_tables T) {
+    static_assert(!X32 || (is_e<MODE> && XL && NC > 1 && CG == 1), "word rows: base and Monte, several chains per lane");
+    static_assert(RG == 1 || X32, "row groups share word rows");
     extern __shared__ __align__(16) char lds[];
     // a widened launch: the workgroups between the working ones leave at once
     if (blockIdx.x & ((1u << a.xcd_sh) - 1u)) return;
@@ -1314,18 +1812,23 @@ __global__ __launch_bounds__(k_block * CG) void k_mm16(mm_args16 a, dev_tables T
     int64_t zw, zx;
     const bool slice_ok = mm_slices(a, z, i12, i13, zw, zx);
     const int lane = (int)(threadIdx.x & 63u);
-    constexpr bool dup = W < 64 && MODE != LNSHIP_SUM32;   // a chain on 64 / W lanes
+        constexpr bool dup = W < 64 && MODE != LNSHIP_SUM32;   // a chain on 64 / W lanes
     const int wr = dup ? lane / (64 / W) : lane;              // the lane's row in the wave
     const int64_t m = W < 64 ? (int64_t)(blockIdx.x >> a.xcd_sh) * (k_block / 64 * W) + (threadIdx.x >> 6) * W + wr
-                             : (int64_t)(blockIdx.x >> a.xcd_sh) * k_block + (threadIdx.x % k_block);
+                             : (int64_t)(blockIdx.x >> a.xcd_sh) * (k_block * RG) + (threadIdx.x % (k_block * RG));
     const bool live = !(W < 64 && !dup && lane >= W) && m < a.M && nc > 0 && slice_ok;
     // one-column launches: the chain's first weights loaded before the
     // tables are staged (their HBM latency passes meanwhile)
     constexpr bool head = NC == 1 && XL;
     mm_head<PF> hw{};
     if (head && live && a.K > 0) hw = mm16_head<PF>(a, m, zw);
-    const red16<MODE> R = stage_for<MODE, NC == 1>(T, lds);
-    uint16_t *xl = reinterpret_cast<uint16_t *>(lds + mm_xl_offset<MODE>());
+    const auto R = [&] {
+        if constexpr (is_e<MODE>) return stage_e<MODE>(T, lds, !a.no_tab);
+        else return stage_for<MODE, NC == 1>(T, lds);
+    }();
+    lfsr8_tab L8{};
+    if (MODE == LNSHIP_MONTE && !a.no_tab) L8 = stage_lfsr8(T, lds + eform<LNSHIP_MONTE>::bytes);
+    uint16_t *xl = reinterpret_cast<uint16_t *>(lds + (is_e<MODE> && a.no_tab ? 0 : mm16_tab_bytes<MODE>()));
     // The RMS_NORM and MUL nodes before the product (norm): each workgroup
     // forms the scales of its own columns' rows, as k_rms16 does: the
     // squares into the activation rows' LDS, then one row's chain per lane
@@ -1335,7 +1838,7 @@ __global__ __launch_bounds__(k_block * CG) void k_mm16(mm_args16 a, dev_tables T
     if (XL && a.norm) {
         const float *xf = a.xf + zx * a.x_slice + nw * a.x_ld;
         const int K = (int)a.K;
-        for (int e = threadIdx.x; e < ncw * K; e += k_block * CG) {
+        for (int e = threadIdx.x; e < ncw * K; e += k_block * CG * RG) {
             const int j = e / K, k = e - j * K;
             const uint32_t c = x16_from_f32(T.cvt16, xf[(int64_t)j * a.x_ld + k]);
             xl[j * kp + k] = (uint16_t)x16_mul(c, c);
@@ -1346,9 +1849,15 @@ __global__ __launch_bounds__(k_block * CG) void k_mm16(mm_args16 a, dev_tables T
             uint32_t s = 0;
             if constexpr (MODE == LNSHIP_MONTE)
                 s = lfsr_jump(T, monte_start(T, a.rms_seed, a.state, a.rms_offset), (uint64_t)(nw + j) * (uint64_t)K);
-            typename red16<MODE>::acc_t acc = R.start(0u, s);
-            chain16<red16<MODE>, true>(R, acc, xl + j * kp, 0, K, s);   // squares: positive
-            const uint32_t mean = x16_mul(R.finish(acc) & 0xffffu, a.rms_ik);
+            uint32_t sum;   // of squares: positive
+            if constexpr (is_e<MODE>) {
+                sum = chain_e_pos<MODE, false>(R, 0u, xl + j * kp, 0, K, s);
+            } else {
+                typename red16<MODE>::acc_t acc = R.start(0u, s);
+                chain16<red16<MODE>, true>(R, acc, xl + j * kp, 0, K, s);
+                sum = R.finish(acc);
+            }
+            const uint32_t mean = x16_mul(sum & 0xffffu, a.rms_ik);
             // the epsilon add is a plain xlns16_add in every mode
             if ((int)threadIdx.x < ncw) s_rinv[j] = x16_recip(x16_sqrt(x16_add_g(T.gauss16, mean, a.rms_eps)));
         }
@@ -1361,13 +1870,16 @@ __global__ __launch_bounds__(k_block * CG) void k_mm16(mm_args16 a, dev_tables T
         // The staging with the rms_norm's scale is a loop of its own, so the
         // plain and GLU launches keep theirs as they were.
         const float *xf = a.xf + zx * a.x_slice + nw * a.x_ld;
-        constexpr int nt = k_block * CG, B = 8;
+        constexpr int nt = k_block * CG * RG, B = 8;
         const int kl = (int)a.K - 1;
         auto stage = [&](auto norm_tag) __attribute__((always_inline)) {
             constexpr bool NORM = decltype(norm_tag)::value;
             for (int j = 0; j < NC * CG; j++) {
                 if (kl < 0) {
-                    for (int k = threadIdx.x; k < kp; k += nt) xl[j * kp + k] = 0;
+                    for (int k = threadIdx.x; k < kp; k += nt) {
+                        if constexpr (X32) reinterpret_cast<int32_t *>(xl)[j * kp + k] = 0;
+                        else xl[j * kp + k] = 0;
+                    }
                     continue;
                 }
                 // loads and lookups stay in the row; only the stores are bounded
@@ -1407,14 +1919,23 @@ __global__ __launch_bounds__(k_block * CG) void k_mm16(mm_args16 a, dev_tables T
 #pragma unroll
                     for (int q = 0; q < B; q++) {
                         const int k = k0 + q * nt;
-                        if (k < kp) xl[j * kp + k] = (j < ncw && k <= kl) ? (uint16_t)c[q] : (uint16_t)0;
+                        // (base and Monte: a column past N repeats the last
+                        // one, whose sums stay in the fast form's range)
+                        if constexpr (X32) {
+                            // the word of a code, less the product's offset
+                            if (k < kp)
+                                reinterpret_cast<int32_t *>(xl)[j * kp + k] =
+                                    e_of<is_e<MODE> ? MODE : LNSHIP_BASE>(c[q]) - eform<is_e<MODE> ? MODE : LNSHIP_BASE>::zero;
+                        } else {
+                            if (k < kp) xl[j * kp + k] = ((is_e<MODE> || j < ncw) && k <= kl) ? (uint16_t)c[q] : (uint16_t)0;
+                        }
                     }
                 }
             }
         };
         if (a.norm) stage(std::true_type{});
         else stage(std::false_type{});
-        xl += cg * NC * kp;
+        xl += cg * NC * kp;   // (X32: one group)
     }
     __syncthreads();
 
@@ -1436,7 +1957,9 @@ __global__ __launch_bounds__(k_block * CG) void k_mm16(mm_args16 a, dev_tables T
     }
 
     uint32_t res[NC];
-    mm16_chains<MODE, NC, PF, XL, head>(a, T, R, xl, m, z, zw, zx, n0, nc, res, hw);
+    if constexpr (is_e<MODE> && NC == 1) res[0] = mme_chain1<MODE, PF, XL, head>(a, T, R, L8, xl, m, z, zw, zx, n0, hw);
+    else if constexpr (is_e<MODE>) mme_chains<MODE, NC, PF, XL, X32>(a, T, R, L8, xl, m, z, zw, zx, n0, nc, res);
+    else mm16_chains<MODE, NC, PF, XL, head>(a, T, R, xl, m, z, zw, zx, n0, nc, res, hw);
     if (dup && lane % (64 / W) != 0) return;   // one lane of a chain stores
 #pragma unroll
     for (int j = 0; j < NC; j++)
@@ -1703,7 +2226,7 @@ __global__ __launch_bounds__(k_block * CG) void k_mm32(mm_args32 a, dev_tables T
 // each group of codes arrives in one 16-byte read issued a group ahead.
 // POS: the accumulator and every row[i] are positive (sign bit clear), so the
 // xlns32 sum takes the one-round positive addition.
-template <class RED, bool POS = false>
+template <class RED, bool POS>
 __device__ __forceinline__ void chain16(const RED &R, typename RED::acc_t &acc, const uint16_t *row, int i0, int n,
                                         uint32_t &st) {
     const int g0 = i0 >> 3, gl = (n - 1) >> 3;
@@ -1733,6 +2256,87 @@ __device__ __forceinline__ void chain16(const RED &R, typename RED::acc_t &acc, 
         run(cur, 0, 8);
     }
     if (gl > g0) run(nxt, 0, n - 8 * gl);
+}
+
+// chain16<RED, true> for base and Monte over the one-word adder: the xlns16
+// code of a (+) row[i0] (+) .. (+) row[n-1], every operand a positive code.
+// Blocks of four groups in the fast form, again in the exact one when one
+// left its range (as mme_chain1; positive sums only grow, so a block's ends
+// tell).  st: the LFSR state before the first draw.  POS: the positive
+// table, else the full one.
+template <int MODE, bool POS>
+__device__ __forceinline__ uint32_t chain_e_pos(const red_e<MODE, POS> &R, uint32_t a, const uint16_t *row, int i0,
+                                                int n, uint32_t st) {
+    using E = eform<MODE, POS>;
+    constexpr int PF = 4;
+    const int g0 = i0 >> 3, gl = (n - 1) >> 3;
+    auto ld = [&](int g) { return *reinterpret_cast<const uint4 *>(row + 8 * min(g, gl)); };
+    int32_t acc = (int32_t)((a + E::bias) << E::sh);
+    auto word = [&](uint32_t w, int u) {
+        if constexpr (POS) return (int32_t)(((u & 1) ? w >> 15 : w << 1) & 0x1fffeu);
+        else return (int32_t)((((u & 1) ? w >> 16 : w & 0xffffu) + E::bias) << E::sh);
+    };
+    auto next_draw = [&] {
+        if constexpr (E::monte) st = lfsr_step(st);
+        return st >> 10;
+    };
+    bool exact = false;
+    uint4 cur[PF], nxt[PF];
+#pragma unroll
+    for (int p = 0; p < PF; p++) cur[p] = ld(g0 + 1 + p);
+    // the first group and the last run exact (with their bounds), the blocks
+    // between them fast
+    for (int g = g0, g1 = g0 + 1; g <= gl; g = g1, g1 = min(g + PF, g < gl ? gl : gl + 1)) {
+        bool redo = true;
+        if (g > g0 && g < gl) {
+#pragma unroll
+            for (int p = 0; p < PF; p++) nxt[p] = ld(g + PF + p);
+            if (!exact) {
+                const int32_t a0 = acc;
+                const uint32_t s0 = st;
+                int32_t t = word(cur[0].x, 0);
+#pragma unroll
+                for (int p = 0; p < PF; p++) {
+                    if (g + p >= gl) break;
+                    const uint32_t w[5] = {cur[p].x, cur[p].y, cur[p].z, cur[p].w, cur[p + 1 < PF ? p + 1 : p].x};
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        int32_t tn;
+                        const uint32_t r = next_draw();
+                        R.step1(acc, t, r, [&] {
+                            tn = word(w[(u + 1) >> 1], u + 1);
+                            asm volatile("" ::"v"(tn));
+                        });
+                        t = tn;
+                    }
+                }
+                redo = __any(a0 < E::lo || acc > E::hi) != 0;
+                if (redo) {
+                    acc = a0;
+                    st = s0;
+                }
+            }
+#pragma unroll
+            for (int p = 0; p < PF; p++) cur[p] = nxt[p];
+        }
+        if (redo) {
+#pragma unroll 1
+            for (int q = g; q < g1; q++) {
+                const uint4 v = ld(q);
+                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+                const int u0 = q == g0 ? i0 & 7 : 0, u1 = min(n - 8 * q, 8);
+#pragma unroll
+                for (int u = 0; u < 8; u++)
+                    if (u >= u0 && u < u1) {
+                        int32_t M;
+                        const uint32_t r = next_draw();
+                        R.xstep(acc, word(w[u >> 1], u), r, M);
+                    }
+            }
+            exact = R.g != nullptr || __any(acc < E::lo || acc > E::hi) != 0;
+        }
+    }
+    return red_e<MODE, POS>::finish(acc) & 0xffffu;
 }
 
 // the same over packed xlns32 codes, four per 16-byte group
@@ -1799,6 +2403,23 @@ __device__ __forceinline__ void chain_pos16(const pos_tab &P, uint32_t &l, const
     if (gl > g0) run(nxt, 0, n - 8 * gl);
 }
 
+// The xlns16 code of a (+) row[i0] (+) .. (+) row[n-1] for a row kernel's
+// positive codes (a itself for an empty range), over stage_rows' tables
+template <int MODE, class R>
+__device__ __forceinline__ uint32_t row_sum(const R &red, uint32_t a, const uint16_t *row, int i0, int n, uint32_t st) {
+    if constexpr (is_e<MODE>) {
+        return i0 < n ? chain_e_pos<MODE, true>(red, a, row, i0, n, st) : a;
+    } else if constexpr (MODE == LNSHIP_SUM32) {
+        uint32_t l = a << 16;
+        if (i0 < n) chain_pos16(red, l, row, i0, n);
+        return red16<MODE>{}.finish({l, 0u}) & 0xffffu;
+    } else {
+        auto acc = red.start(a, st);
+        if (i0 < n) chain16<R, true>(red, acc, row, i0, n, st);
+        return red.finish(acc) & 0xffffu;
+    }
+}
+
 // ---- RMS_NORM -------------------------------------------------------------------
 // A workgroup takes rb rows: all threads convert and square into LDS, one lane
 // per row runs the sequential sum, all threads scale.
@@ -1809,8 +2430,7 @@ __global__ __launch_bounds__(k_block) void k_rms16(const float *__restrict__ src
                                                    float eps, uint32_t seed, const uint16_t *state, uint64_t offset,
                                                    dev_tables T) {
     extern __shared__ __align__(16) char lds[];
-    pos_tab P{};
-    const red16<MODE> R = stage_rows<MODE>(T, lds, P);
+    const auto R = stage_rows<MODE>(T, lds);
     uint16_t *sq = reinterpret_cast<uint16_t *>(lds + ((row_tables_bytes<MODE>() + 15) & ~15));
     __shared__ uint32_t s_inv[64];
     const int64_t r0 = (int64_t)blockIdx.x * rb;
@@ -1844,11 +2464,7 @@ __global__ __launch_bounds__(k_block) void k_rms16(const float *__restrict__ src
         uint32_t s = 0;
         if (MODE == LNSHIP_MONTE)
             s = lfsr_jump(T, monte_start(T, seed, state, offset), (uint64_t)(r0 + r) * (uint64_t)ncols);
-        typename red16<MODE>::acc_t acc = R.start(0u, s);
-        // squares: positive
-        if constexpr (MODE == LNSHIP_SUM32) chain_pos16(P, acc.l, sq + r * rs, 0, nc);
-        else chain16<red16<MODE>, true>(R, acc, sq + r * rs, 0, nc, s);
-        const uint32_t sum = R.finish(acc) & 0xffffu;
+        const uint32_t sum = row_sum<MODE>(R, 0u, sq + r * rs, 0, nc, s);   // squares: positive
         const uint32_t mean = x16_mul(sum, x16_from_f32(T.cvt16, 1.0f / (float)ncols));
         const uint32_t e16 = x16_from_f32(T.cvt16, eps);
         // the epsilon add is a plain xlns16_add in every mode
@@ -2085,8 +2701,7 @@ __device__ __forceinline__ const float *mask_row(const sm_args &a, int64_t row) 
 template <int MODE>
 __global__ __launch_bounds__(k_block) void k_softmax16(sm_args a, dev_tables T) {
     extern __shared__ __align__(16) char lds[];
-    pos_tab P{};
-    const red16<MODE> R = stage_rows<MODE>(T, lds, P);
+    const auto R = stage_rows<MODE>(T, lds);
     // the plain xlns16 adder (scale, mask bias, max subtraction) reads the
     // global copy of the Gaussian-log table
     uint16_t *c = reinterpret_cast<uint16_t *>(lds + ((row_tables_bytes<MODE>() + 15) & ~15));
@@ -2182,7 +2797,6 @@ __global__ __launch_bounds__(k_block) void k_softmax16(sm_args a, dev_tables T) 
         if (MODE == LNSHIP_MONTE)
             s = lfsr_jump(T, monte_start(T, a.seed, a.state, a.offset), (uint64_t)(r0 + r) * (uint64_t)(a.n - 1));
         const uint16_t *row = c + r * rs;
-        typename red16<MODE>::acc_t acc = R.start(row[0], s);
         // The entries after the row's last nonzero exp lie after its maximum
         // (whose exp, 1, is nonzero), so the running sum there is at least 1;
         // each of them is an exp of log 0 (masked or underflowed), which every
@@ -2191,11 +2805,8 @@ __global__ __launch_bounds__(k_block) void k_softmax16(sm_args a, dev_tables T) 
         // draws after it are not taken; the next op's start does not depend
         // on them)
         const int n_eff = s_last[r] + 1;
-        if (n_eff > 1) {   // exps: positive
-            if constexpr (MODE == LNSHIP_SUM32) chain_pos16(P, acc.l, row, 1, n_eff);
-            else chain16<red16<MODE>, true>(R, acc, row, 1, n_eff, s);
-        }
-        if ((int)threadIdx.x < nr) s_tot[r] = R.finish(acc) & 0xffffu;
+        const uint32_t tot = row_sum<MODE>(R, row[0], row, 1, n_eff, s);   // exps: positive
+        if ((int)threadIdx.x < nr) s_tot[r] = tot;
     }
     __syncthreads();
     for (int e0 = threadIdx.x; e0 < nel; e0 += B * nt) {
@@ -2672,6 +3283,28 @@ __device__ __forceinline__ void row_chain_x32(const red16<LNSHIP_SUM32> &R, acc_
     }
 }
 
+// row_chain for base and Monte: the sum's code after terms k0 <= k < k1,
+// from the code a (any for k0 = 0).  st: as chain_e
+template <int MODE>
+__device__ __forceinline__ uint32_t row_chain_e(const red_e<MODE> &R, const lfsr8_tab &L8, uint32_t a, uint32_t st,
+                                                const uint16_t *__restrict__ w, int64_t gs, const uint16_t *x, int k0,
+                                                int k1) {
+    if (k1 <= k0) return a;
+    constexpr int PF = 4;
+    const int gl = (k1 - 1) >> 3;
+    auto load_w = [&](int g) { return *reinterpret_cast<const uint4 *>(w + (int64_t)min(g, gl) * gs); };
+    auto load_x = [&](int g) { return *reinterpret_cast<const uint4 *>(x + 8 * min(g, gl)); };
+    auto block = [&](uint4 (&b)[PF], int g) {
+#pragma unroll
+        for (int p = 0; p < PF; p++) b[p] = load_w(g + p);
+    };
+    uint4 wa[PF];
+    block(wa, (k0 >> 3) + 1);
+    int32_t acc = e_of<MODE>(a);
+    chain_e<MODE, PF>(R, L8, acc, st, k0, k1, load_w(k0 >> 3), wa, block, load_w, load_x);
+    return red_e<MODE>::finish(acc) & 0xffffu;
+}
+
 template <int MODE>
 __device__ __forceinline__ void row_chain(const red16<MODE> &R, typename red16<MODE>::acc_t &acc, uint32_t &st,
                                           const uint16_t *__restrict__ w, int64_t gs, const uint16_t *x, int k0,
@@ -2742,11 +3375,18 @@ __global__ __launch_bounds__(k_block) void k_attn16(attn_args a, dev_tables T) {
     // head hh = s nh + h: query head h of sequence s
     const int hh = attn_head(idle), sqn = hh / a.nh, h = hh - sqn * a.nh, kv = h / a.rep;
     if (idle) return;
-    const red16<MODE> R = stage_for<MODE, true>(T, lds);
+    const auto R = [&] {
+        if constexpr (is_e<MODE>) return stage_e<MODE>(T, lds);
+        else return stage_for<MODE, true>(T, lds);
+    }();
+    lfsr8_tab L8{};
+    if constexpr (MODE == LNSHIP_MONTE) L8 = stage_lfsr8(T, lds + eform<MODE>::bytes);
     const int hd = a.hd, n = a.n_kv, hp = (hd + 7) & ~7, rs = (n + 7) & ~7;
-    uint16_t *xq = reinterpret_cast<uint16_t *>(lds + mm_xl_offset<MODE>());   // the query's codes
-    uint16_t *c = xq + hp;                                                     // scores, then exps
-    uint16_t *pc = c + rs;                                                     // KQV's activation codes
+    uint16_t *xq = reinterpret_cast<uint16_t *>(lds + mm16_tab_bytes<MODE>());   // the query's codes
+    uint16_t *c = xq + hp;                                                       // scores, then exps
+    // KQV's activation codes (base and Monte: in the exps' place, each formed
+    // by the thread that reads its exp, after the sum)
+    uint16_t *pc = is_e<MODE> ? c : c + rs;
     __shared__ int32_t s_max;
     __shared__ uint32_t s_tot, s_tot2;   // the total (sum32: predicted, then the chain's)
     __shared__ float s_part[k_block / 64];
@@ -2779,12 +3419,18 @@ __global__ __launch_bounds__(k_block) void k_attn16(attn_args a, dev_tables T) {
         for (int i = 0; i < 3; i++) ms[i] = monte_start(T, a.mseed[i], a.mstate, a.moff[i]);
     for (int j = threadIdx.x; j < n; j += blockDim.x) {
         uint32_t st = 0;
-        if constexpr (MODE == LNSHIP_MONTE) st = lfsr_jump(T, ms[0], ((uint64_t)hh * n + j) * (uint64_t)(hd - 1));
-        typename red16<MODE>::acc_t acc{};
-        row_chain<MODE>(R, acc, st, kw + (int64_t)j * 8, a.k_gs, xq, 0, hd);
+        if constexpr (MODE == LNSHIP_MONTE) st = lfsr_jump(T, ms[0], ((uint64_t)hh * n + j) * (uint64_t)(hd - 1) + 65534u);
+        uint32_t kq;
+        if constexpr (is_e<MODE>) {
+            kq = row_chain_e<MODE>(R, L8, 0u, st, kw + (int64_t)j * 8, a.k_gs, xq, 0, hd);
+        } else {
+            typename red16<MODE>::acc_t acc{};
+            row_chain<MODE>(R, acc, st, kw + (int64_t)j * 8, a.k_gs, xq, 0, hd);
+            kq = R.finish(acc) & 0xffffu;
+        }
         const float mf = has_mask ? mrow[j] : 0.0f;
         // the score through F32 into xlns16 (the soft_max node reads it so)
-        const uint32_t v = T.rho16[R.finish(acc) & 0xffffu], mk = x16_from_f32(T.cvt16, mf);
+        const uint32_t v = T.rho16[kq], mk = x16_from_f32(T.cvt16, mf);
         const uint32_t vm = x16_mul(v, sc), va = x16_add_g(T.gauss16, vm, mk);
         const bool masked_out = has_mask && (mf <= -3.0e38f || mk == 0xffffu);
         const uint32_t w = v == 0xffffu || masked_out ? 0xffffu : (has_mask && (mk & k16_logmask)) ? va : vm;
@@ -2808,9 +3454,13 @@ __global__ __launch_bounds__(k_block) void k_attn16(attn_args a, dev_tables T) {
     auto sum_chain = [&]() __attribute__((always_inline)) {
         uint32_t st = 0;
         if constexpr (MODE == LNSHIP_MONTE) st = lfsr_jump(T, ms[1], (uint64_t)hh * (uint64_t)(n - 1));
-        typename red16<MODE>::acc_t acc = R.start(c[0], st);
-        if (n_eff > 1) chain16<red16<MODE>, true>(R, acc, c, 1, n_eff, st);
-        return R.finish(acc) & 0xffffu;
+        if constexpr (is_e<MODE>) {
+            return n_eff > 1 ? chain_e_pos<MODE, false>(R, c[0], c, 1, n_eff, st) : (uint32_t)c[0];
+        } else {
+            typename red16<MODE>::acc_t acc = R.start(c[0], st);
+            if (n_eff > 1) chain16<red16<MODE>, true>(R, acc, c, 1, n_eff, st);
+            return R.finish(acc) & 0xffffu;
+        }
     };
     // threads t0, t0 + nt, ...: the largest V log of each dim over the cells
     // past the last nonzero exp
@@ -2845,23 +3495,33 @@ __global__ __launch_bounds__(k_block) void k_attn16(attn_args a, dev_tables T) {
     auto out_chain = [&](int d) __attribute__((always_inline)) {
         const uint32_t p_tail = n_eff < n ? pc[n_eff] & k16_logmask : 0u;
         const uint16_t *vr = vw + (int64_t)d * 8;
-        uint32_t st = 0;
-        if constexpr (MODE == LNSHIP_MONTE) st = lfsr_jump(T, ms[2], ((uint64_t)hh * hd + d) * (uint64_t)(n - 1));
-        typename red16<MODE>::acc_t acc{};
         bool rest = n_eff < n;
-        if (rest && tail_stop) {
-            row_chain<MODE>(R, acc, st, vr, a.v_gs, pc, 0, n_eff);
-            const uint32_t tmax = (uint32_t)min(max((int32_t)(s_vmax[d] + p_tail) - (int32_t)k16_one, 0),
-                                                (int32_t)k16_logmask);
-            if constexpr (MODE == LNSHIP_BASE) rest = acc.l < tmax + (uint32_t)k16_esszer + 1u;
-            // Monte: no draw moves a sum at a distance of k16_mc_end or more
-            else if constexpr (MODE == LNSHIP_MONTE) rest = acc.l < tmax + (uint32_t)k16_mc_end;
-            else rest = acc.l < (tmax << 16) + k32_esszer;   // xlns32 accumulators (sum32, lpvip)
-            if (rest) row_chain<MODE>(R, acc, st, vr, a.v_gs, pc, n_eff, n);
+        const bool stop = rest && tail_stop;
+        const uint32_t tmax = stop ? (uint32_t)min(max((int32_t)(s_vmax[d] + p_tail) - (int32_t)k16_one, 0),
+                                                   (int32_t)k16_logmask) : 0u;
+        if constexpr (is_e<MODE>) {
+            // one draw before term k's group (as chain_e takes it)
+            auto start = [&](int k) {
+                if constexpr (MODE != LNSHIP_MONTE) return 0u;
+                else return lfsr_jump(T, ms[2], ((uint64_t)hh * hd + d) * (uint64_t)(n - 1) + 65534u + (uint64_t)(k & ~7));
+            };
+            uint32_t s = row_chain_e<MODE>(R, L8, 0u, start(0), vr, a.v_gs, pc, 0, stop ? n_eff : n);
+            // (Monte: no draw moves a sum at a distance of k16_mc_end or more)
+            if (stop && (s & k16_logmask) < tmax + (uint32_t)eform<MODE>::far)
+                s = row_chain_e<MODE>(R, L8, s, start(n_eff), vr, a.v_gs, pc, n_eff, n);
+            return s;
         } else {
-            row_chain<MODE>(R, acc, st, vr, a.v_gs, pc, 0, n);
+            uint32_t st = 0;
+            typename red16<MODE>::acc_t acc{};
+            if (stop) {
+                row_chain<MODE>(R, acc, st, vr, a.v_gs, pc, 0, n_eff);
+                rest = acc.l < (tmax << 16) + k32_esszer;   // xlns32 accumulators (sum32, lpvip)
+                if (rest) row_chain<MODE>(R, acc, st, vr, a.v_gs, pc, n_eff, n);
+            } else {
+                row_chain<MODE>(R, acc, st, vr, a.v_gs, pc, 0, n);
+            }
+            return R.finish(acc) & 0xffffu;
         }
-        return R.finish(acc) & 0xffffu;
     };
     // sum32, with a wave beside the output chains' (head_dim <= 192): the
     // output chains start at once from a predicted total while that wave's
@@ -3309,6 +3969,10 @@ static int64_t max_row(int tab_bytes, int elem_bytes) {
     return ((k_lds_bytes - ((tab_bytes + 15) & ~15) - k_lds_static) / 16) * (16 / elem_bytes);
 }
 
+// the longest row an xlns16 row kernel takes
+template <int MODE>
+static int64_t row_limit() { return max_row(MODE == LNSHIP_SUM32 ? k_lds_pos32 : lds_tables_bytes<MODE>(), 2); }
+
 // Rows per workgroup of a row kernel: one chain lane per row, so a block
 // takes as long as one chain plus its element passes over all its rows.
 // The most rows LDS holds decide how many rounds of blocks the GPU needs;
@@ -3472,30 +4136,53 @@ static mm16_shape mm16_choose(int mode, int64_t M, int64_t N, int64_t nslices, i
     return {nc, 1, mm16_xl(mode, nc, kp)};
 }
 
-template <int MODE, int NC, bool XL, int CG, int W = 64>
+template <int MODE, int NC, bool XL, int CG, int W = 64, bool X32 = false, int RG = 1>
 static int launch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslices, int cus, hipStream_t st) {
     // prefetch depth within 128 VGPRs at four waves per SIMD
     constexpr int PF = NC == 1 ? (CG >= 4 ? 4 : 8) : NC == 2 ? 2 : (NC == 4 && CG < 4) ? 2 : 1;
-    const int lds = mm_xl_offset<MODE>() + (XL ? (int)(NC * CG * m.kp * 2) + k_xl_pad : 0);
+    const int rows_lds = XL ? (int)(NC * CG * m.kp * (X32 ? 4 : 2)) + k_xl_pad : 0;
+    const bool no_tab = is_e<MODE> && NC == 1 && mm16_tab_bytes<MODE>() + rows_lds > k_lds_bytes - 1024;
+    const int lds = (no_tab ? 0 : mm16_tab_bytes<MODE>()) + rows_lds;
     static_assert(PF * 16 <= k_xl_pad, "prefetch past the activation rows stays in the padding");
     // weight offsets within a block of PF groups are 32-bit
     if ((uint64_t)m.w_mstride * 16 * PF + (uint64_t)m.M * 16 > 0xffffffffu)
         return fail(LNSHIP_ERANGE, "mul_mat: weight rows too long for 32-bit block offsets%s");
     if (lds > 64 * 1024)
-        if (int rc = set_lds(k_mm16<MODE, NC, PF, XL, CG, W>, lds)) return rc;
-    constexpr int rows = W < 64 ? k_block / 64 * W : k_block;   // rows per workgroup
+        if (int rc = set_lds(k_mm16<MODE, NC, PF, XL, CG, W, X32, RG>, lds)) return rc;
+    constexpr int rows = W < 64 ? k_block / 64 * W : k_block * RG;   // rows per workgroup
     dim3 grid((unsigned)((m.M + rows - 1) / rows), (unsigned)((m.N + NC * CG - 1) / (NC * CG)), (unsigned)nslices);
     if (grid.x > 2147483647u || grid.y > 65535u) return fail(LNSHIP_ERANGE, "mul_mat: grid too large%s");
     mm_args16 mx = m;
+    mx.no_tab = no_tab;
     mx.xcd_sh = MODE == LNSHIP_SUM32 ? xcd_shift((uint64_t)grid.x * grid.y * grid.z, cus) : 0;
     grid.x <<= mx.xcd_sh;
-    hipLaunchKernelGGL((k_mm16<MODE, NC, PF, XL, CG, W>), grid, dim3(k_block * CG), lds, st, mx, T);
+    hipLaunchKernelGGL((k_mm16<MODE, NC, PF, XL, CG, W, X32, RG>), grid, dim3(k_block * CG * RG), lds, st, mx, T);
     LNSHIP_HIP(hipGetLastError());
     return 0;
 }
 
 template <int MODE, int NC, int CG>
 static int launch_mm16_x(const mm_args16 &m, const dev_tables &T, int64_t nslices, bool xl, int cus, hipStream_t st) {
+    if constexpr (is_e<MODE> && NC > 1) {
+        const int64_t lds = mm16_tab_bytes<MODE>() + (int64_t)NC * m.kp * 4 + k_xl_pad;
+        if (xl && lds <= k_lds_bytes - 1024) {
+            // as many row groups as bring a CU to twelve waves, while the
+            // launch still has a workgroup for every CU (K 2048, M 8192, N
+            // 512, with one group: base 3692, Monte 1682 GMAC/s; with this
+            // rule 4220 and 2569)
+            const int64_t per_cu = k_lds_bytes / (lds + 512), cols = (m.N + NC - 1) / NC * nslices;
+            int rg = 1;
+            while (rg < 4 && per_cu * 4 * rg < 12 && (m.M + 2 * rg * k_block - 1) / (2 * rg * k_block) * cols >= cus) rg *= 2;
+            switch (rg) {
+                case 4: return launch_mm16<MODE, NC, true, CG, 64, true, 4>(m, T, nslices, cus, st);
+                case 2: return launch_mm16<MODE, NC, true, CG, 64, true, 2>(m, T, nslices, cus, st);
+                default: return launch_mm16<MODE, NC, true, CG, 64, true>(m, T, nslices, cus, st);
+            }
+        }
+        // rows that fill the LDS (one row per workgroup then)
+        if (xl && mm16_tab_bytes<MODE>() + (int64_t)NC * m.kp * 2 + k_xl_pad > k_lds_bytes - 1024)
+            return launch_mm16<MODE, 1, true, 1>(m, T, nslices, cus, st);
+    }
     return xl ? launch_mm16<MODE, NC, true, CG>(m, T, nslices, cus, st) : launch_mm16<MODE, NC, false, CG>(m, T, nslices, cus, st);
 }
 
@@ -3566,7 +4253,7 @@ static int launch_rms16(const float *src, const float *w, float *dst, int64_t nc
                         hipStream_t st) {
     const int64_t rs = (ncols + 7) & ~(int64_t)7;
     const int rb = rows_per_block(row_tables_bytes<MODE>(), rs, 2, nrows, cus);
-    if (rb < 1) return fail(LNSHIP_ERANGE, "rms_norm: row too long for LDS%s");
+    if (rb < 1 || rs > row_limit<MODE>()) return fail(LNSHIP_ERANGE, "rms_norm: row too long for LDS%s");
     const int lds = ((row_tables_bytes<MODE>() + 15) & ~15) + (int)(rb * rs * 2);
     if (int rc = set_lds(k_rms16<MODE>, lds)) return rc;
     hipLaunchKernelGGL(k_rms16<MODE>, dim3((unsigned)((nrows + rb - 1) / rb)), dim3(k_block), lds, st, src, w, dst,
@@ -3592,10 +4279,17 @@ template <int MODE>
 static int attn16_lds(int64_t hd, int64_t n_kv) {
     return mm_xl_offset<MODE>() + (int)(2 * ((hd + 7) & ~(int64_t)7) + 4 * ((n_kv + 7) & ~(int64_t)7));
 }
+// what a launch takes: base and Monte keep one code per cell, beside larger
+// tables (less than attn16_lds at its limit of cells)
+template <int MODE>
+static int attn16_launch_lds(int64_t hd, int64_t n_kv) {
+    if constexpr (!is_e<MODE>) return attn16_lds<MODE>(hd, n_kv);
+    else return mm16_tab_bytes<MODE>() + (int)(2 * ((hd + 7) & ~(int64_t)7) + 2 * ((n_kv + 7) & ~(int64_t)7));
+}
 
 template <int MODE>
 static int launch_attn16(const attn_args &m, int64_t nh, const dev_tables &T, hipStream_t st) {
-    const int lds = attn16_lds<MODE>(m.hd, m.n_kv);
+    const int lds = attn16_launch_lds<MODE>(m.hd, m.n_kv);
     if (int rc = set_lds(k_attn16<MODE>, lds)) return rc;
     hipLaunchKernelGGL(k_attn16<MODE>, dim3(attn_grid(nh)), dim3(k_block), lds, st, m, T);
     LNSHIP_HIP(hipGetLastError());
@@ -3627,7 +4321,7 @@ template <int MODE>
 static int launch_sm16(sm_args &m, int64_t nrows, const dev_tables &T, int cus, hipStream_t st) {
     const int64_t rs = (m.n + 7) & ~(int64_t)7;
     m.rb = rows_per_block(row_tables_bytes<MODE>(), rs, 2, nrows, cus);
-    if (m.rb < 1) return fail(LNSHIP_ERANGE, "soft_max: row too long for LDS%s");
+    if (m.rb < 1 || rs > row_limit<MODE>()) return fail(LNSHIP_ERANGE, "soft_max: row too long for LDS%s");
     const int lds = ((row_tables_bytes<MODE>() + 15) & ~15) + (int)(m.rb * rs * 2);
     if (int rc = set_lds(k_softmax16<MODE>, lds)) return rc;
     hipLaunchKernelGGL(k_softmax16<MODE>, dim3((unsigned)((nrows + m.rb - 1) / m.rb)), dim3(k_block), lds, st, m, T);
@@ -3898,16 +4592,48 @@ int lnship_init(void) {
     }
     if (int rc = upload(g_host->gauss16, 2 * k16_gauss_n, &T.gauss16)) return rc;
     {
-        // the Monte adder's LDS image: host_tables::gauss16m with db's dither
-        // entries (64 - F, -1) as (-F, 63): the adder then draws 63 - r for
-        // db, so that every entry's second word is a plain mask (0 or 63)
-        std::vector<int32_t> mimg(g_host->gauss16m, g_host->gauss16m + 4 * k16_mc_n);
-        for (int d = 0; d < k16_mc_n; d++)
-            if (mimg[4 * d + 3] == -1) {
-                mimg[4 * d + 2] -= 64;
-                mimg[4 * d + 3] = 63;
+        // the one-word adders' tables (eform): sb(d) in slot 4 d, db(d) in the
+        // slots beside it, exact cancellation in slot 1 (an adjustment that
+        // leaves any sum below zero).  Monte: see red_e::adjusted
+        std::vector<int16_t> eb(eform<LNSHIP_BASE>::bytes / 2, 0);
+        std::vector<int32_t> em(eform<LNSHIP_MONTE>::bytes / 4, 0);
+        for (int d = 0; d <= eform<LNSHIP_BASE>::far; d++) {
+            eb[4 * d] = g_host->gauss16[d];
+            if (d > 0) eb[4 * d - 1] = g_host->gauss16[k16_gauss_n + d];
+            if (d < eform<LNSHIP_BASE>::far) eb[4 * d + 1] = d == 0 ? -32768 : g_host->gauss16[k16_gauss_n + d];
+        }
+        for (int d = 0; d <= eform<LNSHIP_MONTE>::far; d++) {
+            const int32_t *e = g_host->gauss16m + 4 * d;
+            const int32_t db = e[3] == 0 ? e[2] + 64 : e[2];
+            em[4 * d] = e[0];
+            if (d > 0) em[4 * d - 1] = db;
+            if (d < eform<LNSHIP_MONTE>::far) em[4 * d + 1] = d == 0 ? -(1 << 26) : db;
+        }
+        // the positive sums' tables: sb(d) alone (Monte: 64 sb or F)
+        std::vector<int16_t> ebp(eform<LNSHIP_BASE, true>::bytes / 2, 0);
+        std::vector<uint16_t> emp(eform<LNSHIP_MONTE, true>::bytes / 2, 0);
+        for (int d = 0; d <= eform<LNSHIP_BASE, true>::far; d++) ebp[d] = g_host->gauss16[d];
+        for (int d = 0; d <= eform<LNSHIP_MONTE, true>::far; d++) emp[d] = (uint16_t)g_host->gauss16m[4 * d];
+        if (int rc = upload(ebp.data(), ebp.size(), &T.ebp)) return rc;
+        if (int rc = upload(emp.data(), emp.size(), &T.emp)) return rc;
+        if (int rc = upload(eb.data(), eb.size(), &T.eb)) return rc;
+        if (int rc = upload(em.data(), em.size(), &T.em)) return rc;
+        // eight LFSR steps from each byte of the state, then the state eight
+        // steps on (one block: k_lfsr8_bytes)
+        std::vector<uint64_t> l8(k_lfsr8_bytes / 8, 0);
+        uint16_t *t8 = reinterpret_cast<uint16_t *>(l8.data() + 512);
+        for (uint32_t half = 0; half < 2; half++)
+            for (uint32_t b = 0; b < 256; b++) {
+                uint16_t v = (uint16_t)(half ? b << 8 : b);
+                uint64_t draws = 0;
+                for (int k = 0; k < 8; k++) {
+                    v = lnship_lfsr_jump(v, 1);
+                    draws |= (uint64_t)(v >> 10) << (8 * k);
+                }
+                l8[half * 256 + b] = draws;
+                if (!half) t8[b] = v;
             }
-        if (int rc = upload(mimg.data(), mimg.size(), &T.gauss16m)) return rc;
+        if (int rc = upload(l8.data(), l8.size(), &T.lfsr8)) return rc;
     }
     if (int rc = upload(g_host->exp16, 1u << 16, &T.exp16)) return rc;
     if (int rc = upload(g_host->lpdb, 3 * k_lp_n, &T.lpdb)) return rc;
@@ -4657,10 +5383,10 @@ int64_t lnship_max_row(int which, int mode) {
     }
     if (which != 0 && which != 1) return 0;
     switch (mode) {
-        case LNSHIP_BASE: return max_row(row_tables_bytes<LNSHIP_BASE>(), 2);
-        case LNSHIP_MONTE: return max_row(row_tables_bytes<LNSHIP_MONTE>(), 2);
-        case LNSHIP_LPVIP: return max_row(row_tables_bytes<LNSHIP_LPVIP>(), 2);
-        case LNSHIP_SUM32: return max_row(row_tables_bytes<LNSHIP_SUM32>(), 2);
+        case LNSHIP_BASE: return row_limit<LNSHIP_BASE>();
+        case LNSHIP_MONTE: return row_limit<LNSHIP_MONTE>();
+        case LNSHIP_LPVIP: return row_limit<LNSHIP_LPVIP>();
+        case LNSHIP_SUM32: return row_limit<LNSHIP_SUM32>();
         default: return 0;
     }
 }
