@@ -1868,16 +1868,18 @@ __device__ __forceinline__ uint32_t mme_chain1(const mm_args16 &a, const dev_tab
 // X32 (base and Monte, several columns): the activation rows are staged as the
 // one-word adders' words, 4 bytes each, where they fit LDS; RG groups of
 // k_block rows then share them, so that long rows leave room for enough waves
-template <int MODE, int NC, int PF, bool XL, int CG, int W = 64, bool X32 = false, int RG = 1>
-__global__ __launch_bounds__(k_block *CG *RG) void k_mm16(mm_args16 a, dev_tables T) {
+// RB: rows of a column group (k_block, or 64 for column groups of one wave)
+template <int MODE, int NC, int PF, bool XL, int CG, int W = 64, bool X32 = false, int RG = 1, int RB = k_block>
+__global__ __launch_bounds__(RB *CG *RG) void k_mm16(mm_args16 a, dev_tables T) {
     static_assert(!X32 || (is_e<MODE> && XL && NC > 1 && CG == 1), "word rows: base and Monte, several chains per lane");
     static_assert(RG == 1 || X32, "row groups share word rows");
+    static_assert(RB == k_block || (W == 64 && RG == 1), "whole waves");
     extern __shared__ __align__(16) char lds[];
     // a widened launch: the workgroups between the working ones leave at once
     if (blockIdx.x & ((1u << a.xcd_sh) - 1u)) return;
     // CG column groups of k_block lanes each share the staged tables: group
     // c takes columns [nw + c NC, nw + (c + 1) NC) of the same k_block rows
-    const int cg = CG == 1 ? 0 : (int)(threadIdx.x / k_block);
+    const int cg = CG == 1 ? 0 : (int)(threadIdx.x / RB);
     const int64_t nw = (int64_t)blockIdx.y * (NC * CG);
     const int64_t n0 = nw + (int64_t)cg * NC;
     const int64_t z = blockIdx.z;
@@ -1891,7 +1893,7 @@ __global__ __launch_bounds__(k_block *CG *RG) void k_mm16(mm_args16 a, dev_table
         constexpr bool dup = W < 64 && MODE != LNSHIP_SUM32;   // a chain on 64 / W lanes
     const int wr = dup ? lane / (64 / W) : lane;              // the lane's row in the wave
     const int64_t m = W < 64 ? (int64_t)(blockIdx.x >> a.xcd_sh) * (k_block / 64 * W) + (threadIdx.x >> 6) * W + wr
-                             : (int64_t)(blockIdx.x >> a.xcd_sh) * (k_block * RG) + (threadIdx.x % (k_block * RG));
+                             : (int64_t)(blockIdx.x >> a.xcd_sh) * (RB * RG) + (threadIdx.x % (RB * RG));
     const bool live = !(W < 64 && !dup && lane >= W) && m < a.M && nc > 0 && slice_ok;
     // one-column launches: the chain's first weights loaded before the
     // tables are staged (their HBM latency passes meanwhile)
@@ -1914,7 +1916,7 @@ __global__ __launch_bounds__(k_block *CG *RG) void k_mm16(mm_args16 a, dev_table
     if (XL && a.norm) {
         const float *xf = a.xf + zx * a.x_slice + nw * a.x_ld;
         const int K = (int)a.K;
-        for (int e = threadIdx.x; e < ncw * K; e += k_block * CG * RG) {
+        for (int e = threadIdx.x; e < ncw * K; e += RB * CG * RG) {
             const int j = e / K, k = e - j * K;
             const uint32_t c = x16_from_f32(T.cvt16, xf[(int64_t)j * a.x_ld + k]);
             xl[j * kp + k] = (uint16_t)x16_mul(c, c);
@@ -1946,7 +1948,7 @@ __global__ __launch_bounds__(k_block *CG *RG) void k_mm16(mm_args16 a, dev_table
         // The staging with the rms_norm's scale is a loop of its own, so the
         // plain and GLU launches keep theirs as they were.
         const float *xf = a.xf + zx * a.x_slice + nw * a.x_ld;
-        constexpr int nt = k_block * CG * RG, B = 8;
+        constexpr int nt = RB * CG * RG, B = 8;
         const int kl = (int)a.K - 1;
         auto stage = [&](auto norm_tag) __attribute__((always_inline)) {
             constexpr bool NORM = decltype(norm_tag)::value;
@@ -2085,8 +2087,9 @@ __device__ __forceinline__ uint32_t x32_silu(uint32_t x) {
 // (one column per workgroup), its nodes before the product with it (the
 // rms_norm and norm MUL, or the swiglu), exactly as they run apart: F32
 // between the nodes, each converted as the next node converts it
-template <int NC, int PF, int CG, int W = 64, bool XL = false>
-__global__ __launch_bounds__(k_block * CG) void k_mm32(mm_args32 a, dev_tables T) {
+// RB: as k_mm16
+template <int NC, int PF, int CG, int W = 64, bool XL = false, int RB = k_block>
+__global__ __launch_bounds__(RB *CG) void k_mm32(mm_args32 a, dev_tables T) {
     static_assert(!XL || (NC == 1 && CG == 1), "XL launches take one column per workgroup");
     extern __shared__ __align__(16) char lds[];
     if (blockIdx.x & ((1u << a.xcd_sh) - 1u)) return;   // as in k_mm16
@@ -2144,10 +2147,10 @@ __global__ __launch_bounds__(k_block * CG) void k_mm32(mm_args32 a, dev_tables T
         }
     }
     __syncthreads();
-    const int cg = CG == 1 ? 0 : (int)(threadIdx.x / k_block);
+    const int cg = CG == 1 ? 0 : (int)(threadIdx.x / RB);
     const int lane = (int)(threadIdx.x & 63u);
     const int64_t m = W < 64 ? (int64_t)(blockIdx.x >> a.xcd_sh) * (k_block / 64 * W) + (threadIdx.x >> 6) * W + lane
-                             : (int64_t)(blockIdx.x >> a.xcd_sh) * k_block + (threadIdx.x % k_block);
+                             : (int64_t)(blockIdx.x >> a.xcd_sh) * RB + (threadIdx.x % RB);
     const int64_t n0 = ((int64_t)blockIdx.y * CG + cg) * NC;
     if ((W < 64 && lane >= W) || m >= a.M || n0 >= a.N) return;
     const int64_t z = blockIdx.z;
@@ -4139,31 +4142,42 @@ static int mm16_nc(int mode, int64_t M, int64_t N, int64_t nslices, int64_t kp, 
 struct mm16_shape {
     int nc, cg;   // columns per lane, column groups per workgroup
     bool xl;      // activations converted into LDS inside the kernel
+    int rb;       // rows of a column group
 };
 
 // The xlns32 tables leave room for one workgroup per CU, so the sum32 and
-// xlns32 GEMVs take their waves per SIMD from column groups.  Time per k of a
+// xlns32 GEMVs take their waves per SIMD from column groups, of k_block rows
+// or of one wave's 64 (a matrix of few rows, as attention's value product,
+// would leave most waves of a k_block group without rows: M 64, K 256, N 203,
+// 9 slices 138 us in groups of 256, 51 us in groups of 64; 576 x 576 by
+// 201 columns 160 -> 94 us).  Time per k of a
 // shape is rounds x (chains per SIMD) x (time per chain step at that many
 // waves per SIMD); measured on MI355X, a chain step costs 166 ns with one
 // wave and one chain (the adder's latency), 148 ns with one wave of several
-// chains, 103 ns at two waves and 85 ns at four (the VALU issue rate of 49
-// instructions).
+// chains, 103 ns at two waves, 91 at three and 85 ns at four (the VALU issue
+// rate of 49 instructions).
+// max_nc: 8 (sum32, whose launches may stage their rows in LDS) or 4 (xlns32)
 static mm16_shape mm_shape_x32(int64_t M, int64_t N, int64_t nslices, int64_t kp, int cus, int max_nc) {
     // (one wave of several chains, or two waves of two or more, never wins)
-    static const int shapes[][2] = {{1, 1}, {1, 2}, {1, 4}, {2, 4}, {4, 4}, {8, 4}};
-    const int64_t wg_m = (M + k_block - 1) / k_block;
-    mm16_shape best{1, 1, mm16_xl(LNSHIP_SUM32, 1, kp)};
+    static const int shapes[][3] = {{1, 1, k_block}, {1, 2, k_block}, {1, 4, k_block}, {2, 4, k_block}, {4, 4, k_block},
+                                    {8, 4, k_block}, {1, 8, 64}, {1, 12, 64}, {1, 16, 64}, {2, 16, 64}, {4, 16, 64}};
+    mm16_shape best{1, 1, mm16_xl(LNSHIP_SUM32, 1, kp), k_block};
     int64_t best_cost = -1;
     for (const auto &sh : shapes) {
-        const int nc = sh[0], cg = sh[1];
+        const int nc = sh[0], cg = sh[1], rb = sh[2], waves = cg * rb / k_block;   // per SIMD
         if ((nc * cg > 1 && nc * cg > N) || nc > max_nc) continue;
-        const int64_t wgs = wg_m * ((N + nc * cg - 1) / (nc * cg)) * nslices;
+        const bool xl = mm16_xl(LNSHIP_SUM32, nc * cg, kp);
+        // a group of 64 rows in place of one of 256 only where it needs no
+        // scratch that the other did without
+        if (rb == 64 && max_nc == 8 && best.xl && !xl) continue;
+        const int64_t wgs = (M + rb - 1) / rb * ((N + nc * cg - 1) / (nc * cg)) * nslices;
         const int64_t rounds = (wgs + std::max(cus, 1) - 1) / std::max(cus, 1);
-        const int64_t step = cg == 1 ? (nc == 1 ? 166 : 148) : cg == 2 ? 103 : 85;
-        const int64_t cost = rounds * cg * nc * step;
-        // ties go to more columns per workgroup (one weight decode serves them)
-        if (best_cost < 0 || cost <= best_cost) {
-            best = {nc, cg, mm16_xl(LNSHIP_SUM32, nc * cg, kp)};
+        const int64_t step = waves == 1 ? (nc == 1 ? 166 : 148) : waves == 2 ? 103 : waves == 3 ? 91 : 85;
+        const int64_t cost = rounds * waves * nc * step;
+        // ties go to more columns per workgroup (one weight decode serves
+        // them), and to groups of k_block rows
+        if (best_cost < 0 || (rb == 64 ? cost < best_cost : cost <= best_cost)) {
+            best = {nc, cg, xl, rb};
             best_cost = cost;
         }
     }
@@ -4214,13 +4228,13 @@ static uint32_t xcd_shift(uint64_t wgs, int cus) {
 static mm16_shape mm16_choose(int mode, int64_t M, int64_t N, int64_t nslices, int64_t kp, int cus) {
     if (mode == LNSHIP_SUM32) return mm_shape_x32(M, N, nslices, kp, cus, 8);
     const int nc = mm16_nc(mode, M, N, nslices, kp, cus);
-    return {nc, 1, mm16_xl(mode, nc, kp)};
+    return {nc, 1, mm16_xl(mode, nc, kp), k_block};
 }
 
-template <int MODE, int NC, bool XL, int CG, int W = 64, bool X32 = false, int RG = 1>
+template <int MODE, int NC, bool XL, int CG, int W = 64, bool X32 = false, int RG = 1, int RB = k_block>
 static int launch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslices, int cus, hipStream_t st) {
     // prefetch depth within 128 VGPRs at four waves per SIMD
-    constexpr int PF = NC == 1 ? (CG >= 4 ? 4 : 8) : NC == 2 ? 2 : (NC == 4 && CG < 4) ? 2 : 1;
+    constexpr int PF = NC == 1 ? (CG * RB >= 4 * k_block ? 4 : 8) : NC == 2 ? 2 : (NC == 4 && CG < 4) ? 2 : 1;
     const int rows_lds = XL ? (int)(NC * CG * m.kp * (X32 ? 4 : 2)) + k_xl_pad : 0;
     const bool no_tab = is_e<MODE> && NC == 1 && mm16_tab_bytes<MODE>() + rows_lds > k_lds_bytes - 1024;
     const int lds = (no_tab ? 0 : mm16_tab_bytes<MODE>()) + rows_lds;
@@ -4229,20 +4243,20 @@ static int launch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslices,
     if ((uint64_t)m.w_mstride * 16 * PF + (uint64_t)m.M * 16 > 0xffffffffu)
         return fail(LNSHIP_ERANGE, "mul_mat: weight rows too long for 32-bit block offsets%s");
     if (lds > 64 * 1024)
-        if (int rc = set_lds(k_mm16<MODE, NC, PF, XL, CG, W, X32, RG>, lds)) return rc;
-    constexpr int rows = W < 64 ? k_block / 64 * W : k_block * RG;   // rows per workgroup
+        if (int rc = set_lds(k_mm16<MODE, NC, PF, XL, CG, W, X32, RG, RB>, lds)) return rc;
+    constexpr int rows = W < 64 ? k_block / 64 * W : RB * RG;   // rows per workgroup
     dim3 grid((unsigned)((m.M + rows - 1) / rows), (unsigned)((m.N + NC * CG - 1) / (NC * CG)), (unsigned)nslices);
     if (grid.x > 2147483647u || grid.y > 65535u) return fail(LNSHIP_ERANGE, "mul_mat: grid too large%s");
     mm_args16 mx = m;
     mx.no_tab = no_tab;
     mx.xcd_sh = MODE == LNSHIP_SUM32 ? xcd_shift((uint64_t)grid.x * grid.y * grid.z, cus) : 0;
     grid.x <<= mx.xcd_sh;
-    hipLaunchKernelGGL((k_mm16<MODE, NC, PF, XL, CG, W, X32, RG>), grid, dim3(k_block * CG * RG), lds, st, mx, T);
+    hipLaunchKernelGGL((k_mm16<MODE, NC, PF, XL, CG, W, X32, RG, RB>), grid, dim3(RB * CG * RG), lds, st, mx, T);
     LNSHIP_HIP(hipGetLastError());
     return 0;
 }
 
-template <int MODE, int NC, int CG>
+template <int MODE, int NC, int CG, int RB = k_block>
 static int launch_mm16_x(const mm_args16 &m, const dev_tables &T, int64_t nslices, bool xl, int cus, hipStream_t st) {
     if constexpr (is_e<MODE> && NC > 1) {
         const int64_t lds = mm16_tab_bytes<MODE>() + (int64_t)NC * m.kp * 4 + k_xl_pad;
@@ -4264,7 +4278,8 @@ static int launch_mm16_x(const mm_args16 &m, const dev_tables &T, int64_t nslice
         if (xl && mm16_tab_bytes<MODE>() + (int64_t)NC * m.kp * 2 + k_xl_pad > k_lds_bytes - 1024)
             return launch_mm16<MODE, 1, true, 1>(m, T, nslices, cus, st);
     }
-    return xl ? launch_mm16<MODE, NC, true, CG>(m, T, nslices, cus, st) : launch_mm16<MODE, NC, false, CG>(m, T, nslices, cus, st);
+    return xl ? launch_mm16<MODE, NC, true, CG, 64, false, 1, RB>(m, T, nslices, cus, st)
+              : launch_mm16<MODE, NC, false, CG, 64, false, 1, RB>(m, T, nslices, cus, st);
 }
 
 template <int MODE>
@@ -4273,6 +4288,13 @@ static int dispatch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslice
     if constexpr (MODE == LNSHIP_SUM32) {
         // column groups: more waves per SIMD where the tables allow one
         // workgroup per CU
+        if (sh.rb == 64) switch (sh.nc * 100 + sh.cg) {
+                case 108: return launch_mm16_x<MODE, 1, 8, 64>(m, T, nslices, sh.xl, cus, st);
+                case 112: return launch_mm16_x<MODE, 1, 12, 64>(m, T, nslices, sh.xl, cus, st);
+                case 116: return launch_mm16_x<MODE, 1, 16, 64>(m, T, nslices, sh.xl, cus, st);
+                case 216: return launch_mm16_x<MODE, 2, 16, 64>(m, T, nslices, sh.xl, cus, st);
+                default: return launch_mm16_x<MODE, 4, 16, 64>(m, T, nslices, sh.xl, cus, st);
+            }
         switch (sh.nc * 10 + sh.cg) {
             case 12: return launch_mm16_x<MODE, 1, 2>(m, T, nslices, sh.xl, cus, st);
             case 14: return launch_mm16_x<MODE, 1, 4>(m, T, nslices, sh.xl, cus, st);
@@ -4311,19 +4333,19 @@ static int64_t mm32_lds(bool xl, int64_t kp) { return k_lds_tab32 + (xl ? kp * 4
 // whether an XL launch of rows of kp codes fits LDS
 static bool mm32_xl_fits(int64_t kp) { return mm32_lds(true, kp) <= k_lds_bytes - k_lds_static; }
 
-template <int NC, int CG, int W = 64, bool XL = false>
+template <int NC, int CG, int W = 64, bool XL = false, int RB = k_block>
 static int launch_mm32(const mm_args32 &m, const dev_tables &T, int64_t nslices, int cus, hipStream_t st) {
     // prefetch depth within 128 VGPRs at four waves per SIMD
-    constexpr int PF = NC == 1 ? (CG >= 4 ? 2 : 4) : 1;
+    constexpr int PF = NC == 1 ? (CG * RB >= 4 * k_block ? 2 : 4) : 1;
     const int lds = (int)mm32_lds(XL, m.kp);
-    if (int rc = set_lds(k_mm32<NC, PF, CG, W, XL>, lds)) return rc;
-    constexpr int rows = W < 64 ? k_block / 64 * W : k_block;   // rows per workgroup
+    if (int rc = set_lds(k_mm32<NC, PF, CG, W, XL, RB>, lds)) return rc;
+    constexpr int rows = W < 64 ? k_block / 64 * W : RB;   // rows per workgroup
     dim3 grid((unsigned)((m.M + rows - 1) / rows), (unsigned)((m.N + NC * CG - 1) / (NC * CG)), (unsigned)nslices);
     if (grid.x > 2147483647u || grid.y > 65535u) return fail(LNSHIP_ERANGE, "mul_mat: grid too large%s");
     mm_args32 mx = m;
     mx.xcd_sh = xcd_shift((uint64_t)grid.x * grid.y * grid.z, cus);
     grid.x <<= mx.xcd_sh;
-    hipLaunchKernelGGL((k_mm32<NC, PF, CG, W, XL>), grid, dim3(k_block * CG), lds, st, mx, T);
+    hipLaunchKernelGGL((k_mm32<NC, PF, CG, W, XL, RB>), grid, dim3(RB * CG), lds, st, mx, T);
     LNSHIP_HIP(hipGetLastError());
     return 0;
 }
@@ -4982,6 +5004,13 @@ static int mul_mat32_staged(device_state *s, const lnship_mul_mat_args *a, void 
                 wms, a->w_slice ? a->w_slice : kp * wms, dld, a->dst_slice ? a->dst_slice : a->N * dld};
     m.resid = a->residual;
     const mm16_shape sh = mm_shape_x32(m.M, m.N, nslices, kp, s->cus, 4);
+    if (sh.rb == 64) switch (sh.nc * 100 + sh.cg) {
+            case 108: return launch_mm32<1, 8, 64, false, 64>(m, s->T, nslices, s->cus, st);
+            case 112: return launch_mm32<1, 12, 64, false, 64>(m, s->T, nslices, s->cus, st);
+            case 116: return launch_mm32<1, 16, 64, false, 64>(m, s->T, nslices, s->cus, st);
+            case 216: return launch_mm32<2, 16, 64, false, 64>(m, s->T, nslices, s->cus, st);
+            default: return launch_mm32<4, 16, 64, false, 64>(m, s->T, nslices, s->cus, st);
+        }
     switch (sh.nc * 10 + sh.cg) {
         case 12: return launch_mm32<1, 2>(m, s->T, nslices, s->cus, st);
         case 14: return launch_mm32<1, 4>(m, s->T, nslices, s->cus, st);
