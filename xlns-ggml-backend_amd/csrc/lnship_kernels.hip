@@ -763,32 +763,98 @@ struct red16<LNSHIP_LPVIP> {
     __device__ __forceinline__ acc_t start(uint32_t v, uint32_t &) const {
         return {(v & k16_logmask) << 16, (v & k16_sign) << 16};
     }
-    // lpvip_sb and lpvip_db formed side by side, without branches, but for
-    // the FP64 Gaussian log (opposite signs below one binade), which only
-    // lanes that need it run; exact cancellation (d = 0, opposite signs)
-    // gives +0
+    // An addition before its exact branch: the larger log, its sign, the
+    // distance, Mitchell's adjustment, and whether the exact one takes its
+    // place (opposite signs below one binade, exact cancellation included)
+    struct mid {
+        uint32_t mx, s, d;
+        int32_t adj;
+        bool near;
+    };
+    // (tl, ts at the xlns32 positions.)  Mitchell's antilog of the distance,
+    // u = (2^24 - (d mod 2^23)) >> (d / 2^23 + 1) (0 from 24 binades on, to
+    // which d is capped: the essential zero), then its correction: u plus
+    // u (2^23 - u) >> 23 times 0x570 / 2^12 for equal signs, the negated sum of
+    // u and u^2 >> 23 times 0xB8A / 2^12 for opposite ones; one product chain
+    // for both, its operands picked by the lane mask of opposite signs, all of
+    // 24 bits.
+    __device__ __forceinline__ mid front(const acc_t &a, uint32_t tl, uint32_t ts) const {
+        mid m;
+        const uint32_t dq = min(sad_u32(a.l, tl, 0x800000u), k32_esszer + 0x800000u);   // d + one binade
+        const uint32_t op = (uint32_t)((int32_t)(a.s ^ ts) >> 31);
+        const uint32_t u = (0x1000000u - (dq & 0x7fffffu)) >> (dq >> 23);
+        const uint32_t v = bfi(op, u, 0x800000u - u);
+        const uint32_t p = __builtin_amdgcn_alignbit(mulhi_u24(u, v), mul_u24(u, v), 23);
+        const uint32_t c = bfi(op, 0xB8Au, 0x570u);
+        const uint32_t t = u + __builtin_amdgcn_alignbit(mulhi_u24(p, c), mul_u24(p, c), 12);
+        m.adj = (int32_t)((t ^ op) - op);
+        m.mx = max(a.l, tl);
+        m.s = bfi(tl - a.l, a.s, ts);   // the larger operand's sign
+        m.d = dq - 0x800000u;
+        m.near = (dq | ~op) < 0x1000000u;
+        return m;
+    }
+    // the exact adjustment of a near distance (d = 0: one that leaves any log
+    // below 0)
+    __device__ __forceinline__ int32_t exact(uint32_t d) const { return d == 0 ? INT32_MIN : lpvip_db_near(lp, d); }
+    // (the sum is at least 0, at most the largest log; exact cancellation is +0)
+    __device__ __forceinline__ void back(acc_t &a, const mid &m) const {
+        a.l = (uint32_t)max(__builtin_elementwise_add_sat((int32_t)m.mx, m.adj), 0);
+        a.s = m.s;
+    }
+    // One addition; only lanes that need it run the FP64 branch
     __device__ __forceinline__ void add_ls(acc_t &a, uint32_t tl16, uint32_t ts16, uint32_t &) const {
-        const uint32_t tl = tl16 << 16, ts = ts16 << 16;
-        const uint32_t mx = max(a.l, tl), d = mx - min(a.l, tl);
-        const uint32_t sgn = a.l > tl ? a.s : ts;
-        const bool usedb = (a.s ^ ts) != 0;
-        // Mitchell's antilog of -d (0 from 31 binades on), then sb's and db's
-        // corrections of it, all products of 24-bit operands (u <= 2^23):
-        // u (2^23 - u) >> 23 < 2^21, so its product with 0x2B8 fits 32 bits;
-        // u^2 >> 23 <= 2^23, its product with 0xB8A taken as 48 bits
-        const uint32_t u = ((0x1000000u - (d & 0x7fffffu)) >> 1) >> min(d >> 23, 31u);
-        const uint32_t pc = (uint32_t)(((uint64_t)u * (uint64_t)(0x800000u - u)) >> 23);
-        const uint32_t pq = (uint32_t)(((uint64_t)u * u) >> 23);
-        const int32_t sb = (int32_t)(u + (mul_u24(pc, 0x2B8u) >> 11));
-        const int32_t dbm = -(int32_t)(u + __builtin_amdgcn_alignbit(mulhi_u24(pq, 0xB8Au), mul_u24(pq, 0xB8Au), 12));
-        int32_t adj = usedb ? dbm : sb;
-        if (usedb && d - 1u < 0x7fffffu) adj = lpvip_db_near(lp, d);
-        adj = d < k32_esszer ? adj : 0;
-        const uint32_t s = mx + (uint32_t)adj;
-        const uint32_t l = (s & k32_sign) ? ((s & k32_one) ? 0u : k32_logmask) : s;
-        const bool cancel = d == 0 && usedb;
-        a.l = cancel ? 0u : l;
-        a.s = cancel ? 0u : sgn;
+        mid m = front(a, tl16 << 16, ts16 << 16);
+        if (m.near) {
+            m.adj = exact(m.d);
+            if (m.d == 0) m.s = 0;
+        }
+        back(a, m);
+    }
+    // One addition to each of NC chains of a lane.  Opposite signs below one
+    // binade come up in 2-3 % of the additions, so nearly every wave has a lane
+    // in the exact branch (70 instructions) at every one: the wave gathers the
+    // distances of all its chains' near additions in LDS (slots: 64 NC words of
+    // its own), evaluates up to 64 of them at once, and hands them back.  K
+    // 2048, M 8192, N 512: 832 -> 1205 GMAC/s, with the shorter Mitchell part
+    // (which alone took the single chain's step from 138 to 89 ns).
+    template <int NC>
+    __device__ __forceinline__ void add_many(acc_t (&a)[NC], const uint32_t (&tl)[NC], const uint32_t (&ts)[NC],
+                                             uint32_t *slots) const {
+        mid m[NC];
+        uint32_t at[NC], n = 0;
+#pragma unroll
+        for (int j = 0; j < NC; j++) {
+            m[j] = front(a[j], tl[j], ts[j]);
+            const uint64_t mask = __ballot(m[j].near);
+            at[j] = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, n));
+            n += (uint32_t)__popcll(mask);
+        }
+        if (n != 0) {   // wave-uniform
+#pragma unroll
+            for (int j = 0; j < NC; j++)
+                if (m[j].near) slots[at[j]] = m[j].d;
+            __builtin_amdgcn_wave_barrier();   // (a wave's LDS operations complete in order)
+            // the wave's active lanes (those past M have left), in rank order
+            const uint64_t act = __ballot(true);
+            const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(act >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)act, 0u));
+            for (uint32_t r = 0; r < n; r += (uint32_t)__popcll(act)) {
+                const uint32_t i = min(r + rank, n - 1u);
+                const int32_t e = exact(slots[i]);
+                __builtin_amdgcn_wave_barrier();
+                if (r + rank < n) slots[i] = (uint32_t)e;
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int j = 0; j < NC; j++)
+                if (m[j].near) {
+                    m[j].adj = (int32_t)slots[at[j]];
+                    if (m[j].adj == INT32_MIN) m[j].s = 0;
+                }
+            __builtin_amdgcn_wave_barrier();
+        }
+#pragma unroll
+        for (int j = 0; j < NC; j++) back(a[j], m[j]);
     }
     __device__ __forceinline__ void add(acc_t &a, uint32_t v, uint32_t &st) const { add_ls(a, v & k16_logmask, v & k16_sign, st); }
     // add() of a positive v to a positive sum: sb only, the sign stays +
@@ -1178,6 +1244,8 @@ constexpr int mm_xl_offset() { return (lds_tables_bytes<MODE>() + 15) & ~15; }
 // k_mm16's own tables: the one-word adders' for base and Monte, with the LFSR
 // tables when a lane runs several Monte chains
 constexpr int k_lfsr8_bytes = 2 * 256 * 8 + 256 * 2;
+// (lpvip: lp_slots per wave beside the tables when a lane runs several chains)
+constexpr int lp_slot_bytes(int nc) { return nc > 1 ? k_block / 64 * 64 * nc * 4 : 0; }
 template <int MODE>
 constexpr int mm16_tab_bytes() {
     if constexpr (is_e<MODE>) return eform<MODE>::bytes + (MODE == LNSHIP_MONTE ? k_lfsr8_bytes : 0);
@@ -1230,7 +1298,7 @@ template <int MODE, int NC, int PF, bool XL, bool HEAD = false>
 __device__ __forceinline__ void mm16_chains(const mm_args16 &a, const dev_tables &T, const red16<MODE> &R,
                                             const uint16_t *xl, int64_t m, int64_t z, int64_t zw, int64_t zx,
                                             int64_t n0, int nc, uint32_t (&res)[NC],
-                                            const mm_head<PF> &head = mm_head<PF>{}) {
+                                            const mm_head<PF> &head = mm_head<PF>{}, uint32_t *slots = nullptr) {
     const int kp = (int)a.kp;
     const uint16_t *ws = a.w + zw * a.w_slice + m * 8;
     const uint16_t *xs = a.x + (zx * a.N + n0) * a.kp;
@@ -1397,19 +1465,33 @@ __device__ __forceinline__ void mm16_chains(const mm_args16 &a, const dev_tables
             }
             return;
         }
+        // lpvip, several chains per lane: the products as sum32's
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-            if (u >= u0 && u < u1) {
-                const uint32_t wv = half16(ww[u >> 1], u & 1);
-                const uint32_t wl = wv & k16_logmask;
+        for (int i = 0; i < 4; i++) {
+            if (2 * i + 1 < u0 || 2 * i >= u1) continue;
+            const uint32_t wb = pk_sub_u16(ww[i] & k_lm, 0x40004000u);
+            uint32_t pl[NC], ps[NC];
+#pragma unroll
+            for (int j = 0; j < NC; j++) {
+                const uint32_t xv = i == 0 ? xq[j].x : i == 1 ? xq[j].y : i == 2 ? xq[j].z : xq[j].w;
+                pl[j] = pk_add_sat_nonneg_i16(wb, xv & k_lm);
+                ps[j] = ww[i] ^ xv;
+            }
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int u = 2 * i + h;
+                if (u < u0 || u >= u1) continue;
+                uint32_t tl[NC], ts[NC];
 #pragma unroll
                 for (int j = 0; j < NC; j++) {
-                    const uint32_t xv = half16(u < 2 ? xq[j].x : u < 4 ? xq[j].y : u < 6 ? xq[j].z : xq[j].w, u & 1);
-                    const int32_t l = (int32_t)wl + (int32_t)(xv & k16_logmask) - (int32_t)k16_one;
-                    const uint32_t tl = (uint32_t)min(max(l, 0), (int32_t)k16_logmask);
-                    const uint32_t ts = (wv ^ xv) & k16_sign;
-                    if (u == 0 && u0 < 0) acc[j] = R.start(ts | tl, st[j]);
-                    else R.add_ls(acc[j], tl, ts, st[j]);
+                    tl[j] = h == 0 ? pl[j] << 16 : pl[j] & k_hi;
+                    ts[j] = h == 0 ? (ps[j] << 16) & k_sg : ps[j] & k_sg;
+                }
+                if (u == 0 && u0 < 0) {
+#pragma unroll
+                    for (int j = 0; j < NC; j++) acc[j] = {tl[j], ts[j]};
+                } else if constexpr (MODE == LNSHIP_LPVIP) {
+                    R.add_many(acc, tl, ts, slots);
                 }
             }
         }
@@ -1921,7 +2003,9 @@ __global__ __launch_bounds__(RB *CG *RG) void k_mm16(mm_args16 a, dev_tables T) 
     }();
     lfsr8_tab L8{};
     if (MODE == LNSHIP_MONTE && !a.no_tab) L8 = stage_lfsr8(T, lds + eform<LNSHIP_MONTE>::bytes);
-    uint16_t *xl = reinterpret_cast<uint16_t *>(lds + (is_e<MODE> && a.no_tab ? 0 : mm16_tab_bytes<MODE>()));
+    constexpr int slot_bytes = MODE == LNSHIP_LPVIP ? lp_slot_bytes(NC) : 0;
+    uint32_t *slots = reinterpret_cast<uint32_t *>(lds + mm16_tab_bytes<MODE>()) + (threadIdx.x >> 6) * (64 * NC);
+    uint16_t *xl = reinterpret_cast<uint16_t *>(lds + (is_e<MODE> && a.no_tab ? 0 : mm16_tab_bytes<MODE>() + slot_bytes));
     // The RMS_NORM and MUL nodes before the product (norm): each workgroup
     // forms the scales of its own columns' rows, as k_rms16 does: the
     // squares into the activation rows' LDS, then one row's chain per lane
@@ -2052,7 +2136,7 @@ __global__ __launch_bounds__(RB *CG *RG) void k_mm16(mm_args16 a, dev_tables T) 
     uint32_t res[NC];
     if constexpr (is_e<MODE> && NC == 1) res[0] = mme_chain1<MODE, PF, XL, head>(a, T, R, L8, xl, m, z, zw, zx, n0, hw);
     else if constexpr (is_e<MODE>) mme_chains<MODE, NC, PF, XL, X32>(a, T, R, L8, xl, m, z, zw, zx, n0, nc, res);
-    else mm16_chains<MODE, NC, PF, XL, head>(a, T, R, xl, m, z, zw, zx, n0, nc, res, hw);
+    else mm16_chains<MODE, NC, PF, XL, head>(a, T, R, xl, m, z, zw, zx, n0, nc, res, hw, slots);
     if (dup && lane % (64 / W) != 0) return;   // one lane of a chain stores
 #pragma unroll
     for (int j = 0; j < NC; j++)
@@ -4266,7 +4350,7 @@ template <int MODE, int NC, bool XL, int CG, int W = 64, bool X32 = false, int R
 static int launch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslices, int cus, hipStream_t st) {
     // prefetch depth within 128 VGPRs at four waves per SIMD
     constexpr int PF = NC == 1 ? (CG * RB >= 4 * k_block ? 4 : 8) : NC == 2 ? 2 : (NC == 4 && CG < 4) ? 2 : 1;
-    const int rows_lds = XL ? (int)(NC * CG * m.kp * (X32 ? 4 : 2)) + k_xl_pad : 0;
+    const int rows_lds = (XL ? (int)(NC * CG * m.kp * (X32 ? 4 : 2)) + k_xl_pad : 0) + (MODE == LNSHIP_LPVIP ? lp_slot_bytes(NC) : 0);
     const bool no_tab = is_e<MODE> && NC == 1 && mm16_tab_bytes<MODE>() + rows_lds > k_lds_bytes - 1024;
     const int lds = (no_tab ? 0 : mm16_tab_bytes<MODE>()) + rows_lds;
     static_assert(PF * 16 <= k_xl_pad, "prefetch past the activation rows stays in the padding");
@@ -4305,8 +4389,11 @@ static int launch_mm16_x(const mm_args16 &m, const dev_tables &T, int64_t nslice
                 default: return launch_mm16<MODE, NC, true, CG, 64, true>(m, T, nslices, cus, st);
             }
         }
-        // rows that fill the LDS (one row per workgroup then)
-        if (xl && mm16_tab_bytes<MODE>() + (int64_t)NC * m.kp * 2 + k_xl_pad > k_lds_bytes - 1024)
+    }
+    if constexpr (NC > 1 && MODE != LNSHIP_SUM32) {
+        // rows that fill the LDS beside what several chains take (one row
+        // per workgroup then)
+        if (xl && mm16_tab_bytes<MODE>() + (MODE == LNSHIP_LPVIP ? lp_slot_bytes(NC) : 0) + (int64_t)NC * m.kp * 2 + k_xl_pad > k_lds_bytes - 1024)
             return launch_mm16<MODE, 1, true, 1>(m, T, nslices, cus, st);
     }
     return xl ? launch_mm16<MODE, NC, true, CG, 64, false, 1, RB>(m, T, nslices, cus, st)
