@@ -80,6 +80,8 @@ def test_products(ln, mode, kind, K, M, N):
                                    (1200, 1030, 530),    # two, ragged
                                    (5000, 300, 2100),    # word rows do not fit: code rows
                                    (9704, 260, 2100),    # nor do eight code rows beside the table
+                                   (30011, 40, 1),       # one column as logs and signs
+                                   (40007, 40, 1),       # as codes: too long for both
                                    (66000, 3, 1)])       # no room for the table (exact steps only)
 def test_workgroup_shapes(ln, mode, K, M, N):
     print(f"\n[shapes] {mode} K={K} M={M} N={N}", flush=True)

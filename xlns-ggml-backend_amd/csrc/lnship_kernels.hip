@@ -431,6 +431,9 @@ __device__ __forceinline__ uint32_t lds_at4(uint32_t a, uint32_t b) {
 // need hazard wait states on gfx950)
 __device__ __forceinline__ uint32_t bfi(uint32_t m, uint32_t a, uint32_t b) { return (a & m) | (b & ~m); }
 
+// the same as one v_bitop3_b32, where the compiler would hoist ~m and use two
+__device__ __forceinline__ uint32_t bfi1(uint32_t m, uint32_t a, uint32_t b) { return __builtin_amdgcn_bitop3_b32(m, a, b, 0xca); }
+
 // All ones where x is negative as a signed value, else 0, as one v_bfe_i32
 // of bit 31 whose width comes from a register (one = 1 in a register the
 // compiler cannot see into).  A plain shift would be folded into a compare
@@ -911,7 +914,7 @@ __device__ __forceinline__ void stage_copy(int4 *dst, const int4 *__restrict__ s
 // run again by the exact form (xstep), which clamps.
 //
 // Measured on MI355X against the clamping adder with log and sign apart: a
-// single chain's step 51 -> 38 ns (base) and 65 -> 49 ns (Monte); the product
+// single chain's step 51 -> 38 ns (base) and 65 -> 46 ns (Monte); the product
 // K 2048, M 8192, N 512 1913 -> 4220 GMAC/s (base), 1341 -> 2569 (Monte).
 //
 // POS: sums of positive terms only (squares, exps): E = 2 log, one 16-bit
@@ -943,12 +946,20 @@ template <int MODE>
 __device__ __forceinline__ void e_pair(uint32_t w, uint32_t x, uint32_t k_lm, uint32_t k_su, uint32_t &lm, uint32_t &sg) {
     lm = (w & k_lm) + (x & k_lm);
     sg = ((w ^ x) >> (15 - (eform<MODE>::sh - 2))) & k_su;
-    asm("" : "+v"(lm), "+v"(sg));   // (opaque: the inserts below stay one instruction each)
 }
 template <int MODE>
 __device__ __forceinline__ void e_words(uint32_t lm, uint32_t sg, uint32_t k_em, int32_t (&t)[2]) {
-    t[0] = (int32_t)bfi(k_em, lm << eform<MODE>::sh, sg);
-    t[1] = (int32_t)bfi(k_em, lm >> (16 - eform<MODE>::sh), sg >> 16);
+    t[0] = (int32_t)bfi1(k_em, lm << eform<MODE>::sh, sg);
+    t[1] = (int32_t)bfi1(k_em, lm >> (16 - eform<MODE>::sh), sg >> 16);
+}
+// the first part with the activations' half of it staged: their logs, and
+// their signs at u's place
+template <int MODE>
+__device__ __forceinline__ void e_pair_split(uint32_t w, uint32_t xlog, uint32_t xsgn, uint32_t k_lm, uint32_t k_su,
+                                             uint32_t &lm, uint32_t &sg) {
+    lm = (w & k_lm) + xlog;
+    // (the masked sign of w) xor xsgn
+    sg = __builtin_amdgcn_bitop3_b32(w >> (15 - (eform<MODE>::sh - 2)), k_su, xsgn, 0x6a);
 }
 struct e_masks {
     uint32_t lm, em, su;
@@ -1777,16 +1788,26 @@ __device__ __forceinline__ void mme_chains(const mm_args16 &a, const dev_tables 
 // it in wa; block(w, g) loads groups g .. g + PF - 1 (past the last: the last
 // again), load_w(g) and load_x(g) a group's weights and activations.  st:
 // Monte's LFSR state one draw before term 8 (k0 / 8)'s.
-template <int MODE, int PF, class B, class W, class X>
+// SPLIT: the activations are staged as two 16-byte halves per group, the logs
+// and the signs at u's place (e_pair_split): an instruction less per term (a
+// Monte step 49 -> 46 ns; base is bound by the path above, 38 ns either way).
+struct e_grp {
+    uint4 q, s;   // codes; or logs and signs
+};
+template <int MODE, int PF, bool SPLIT, class B, class W, class X>
 __device__ __forceinline__ void chain_e(const red_e<MODE> &R, const lfsr8_tab &L8, int32_t &acc, uint32_t st, int k0,
                                         int k1, const uint4 &w0, uint4 (&wa)[PF], B &&block, W &&load_w, X &&load_x) {
     using E = eform<MODE>;
     const int gf = k0 >> 3, full = k1 >> 3, tail = k1 & 7, groups = full + (tail > 0);
     const e_masks km = e_mask_regs<MODE>();
     int32_t mn = E::hi, mx = E::lo;   // the least and largest M
-    auto pair = [&](uint32_t w, uint32_t x, int32_t (&t)[2]) {
+    auto half = [&](uint32_t w, uint32_t x, uint32_t xs, uint32_t &lm, uint32_t &sg) {
+        if constexpr (SPLIT) e_pair_split<MODE>(w, x, xs, km.lm, km.su, lm, sg);
+        else e_pair<MODE>(w, x, km.lm, km.su, lm, sg);
+    };
+    auto pair = [&](uint32_t w, uint32_t x, uint32_t xs, int32_t (&t)[2]) {
         uint32_t lm, sg;
-        e_pair<MODE>(w, x, km.lm, km.su, lm, sg);
+        half(w, x, xs, lm, sg);
         e_words<MODE>(lm, sg, km.em, t);
     };
     // Monte's draws of a group, a byte each, and those of the next one, whose
@@ -1817,16 +1838,17 @@ __device__ __forceinline__ void chain_e(const red_e<MODE> &R, const lfsr8_tab &L
         asm("v_min3_i32 %0, %0, %1, %2" : "+v"(mn) : "v"(Ma), "v"(Mb));
         asm("v_max3_i32 %0, %0, %1, %2" : "+v"(mx) : "v"(Ma), "v"(Mb));
     };
-    auto fast8 = [&](const uint4 &wq, const uint4 &xq, uint32_t wn, uint32_t xn, int u0) __attribute__((always_inline)) {
-        const uint32_t ww[5] = {wq.x, wq.y, wq.z, wq.w, wn}, xx[5] = {xq.x, xq.y, xq.z, xq.w, xn};
+    auto fast8 = [&](const uint4 &wq, const e_grp &x, uint32_t wn, const e_grp &xn, int u0) __attribute__((always_inline)) {
+        const uint32_t ww[5] = {wq.x, wq.y, wq.z, wq.w, wn}, xx[5] = {x.q.x, x.q.y, x.q.z, x.q.w, xn.q.x};
+        const uint32_t xs[5] = {x.s.x, x.s.y, x.s.z, x.s.w, xn.s.x};
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             int32_t tn[2], M0 = E::hi;
             uint32_t lm = 0, sg = 0;
             auto even = [&] {
-                e_pair<MODE>(ww[i + 1], xx[i + 1], km.lm, km.su, lm, sg);
+                half(ww[i + 1], xx[i + 1], xs[i + 1], lm, sg);
                 note();
-                asm volatile("" ::"v"(mn), "v"(mx));
+                asm volatile("" ::"v"(mn), "v"(mx), "v"(lm), "v"(sg));
             };
             if (2 * i >= u0) M0 = R.step1(acc, t0, draw_of(2 * i), even);
             else even();
@@ -1842,14 +1864,15 @@ __device__ __forceinline__ void chain_e(const red_e<MODE> &R, const lfsr8_tab &L
         dr = drn;
     };
     // steps [u0, u1) of a group in the exact form; start: step 0 starts the sum
-    auto exact8 = [&](const uint4 &wq, const uint4 &xq, int u0, int u1, bool start) __attribute__((always_inline)) {
-        const uint32_t ww[4] = {wq.x, wq.y, wq.z, wq.w}, xx[4] = {xq.x, xq.y, xq.z, xq.w};
+    auto exact8 = [&](const uint4 &wq, const e_grp &x, int u0, int u1, bool start) __attribute__((always_inline)) {
+        const uint32_t ww[4] = {wq.x, wq.y, wq.z, wq.w}, xx[4] = {x.q.x, x.q.y, x.q.z, x.q.w};
+        const uint32_t xs[4] = {x.s.x, x.s.y, x.s.z, x.s.w};
         draws(false);
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             if (u < u0 || u >= u1) continue;
             int32_t t[2], M = E::hi;
-            pair(ww[u >> 1], xx[u >> 1], t);
+            pair(ww[u >> 1], xx[u >> 1], xs[u >> 1], t);
             if (u == 0 && start) acc = red_e<MODE>::clamped(t[0]);
             else R.xstep(acc, t[u & 1], draw_of(u), M);
             mn = min(mn, M);
@@ -1878,22 +1901,22 @@ __device__ __forceinline__ void chain_e(const red_e<MODE> &R, const lfsr8_tab &L
                 int32_t t[2];
                 Ma = Mb = E::hi;
                 if (g == gf) {
-                    const uint4 x0 = load_x(gf);
-                    pair(w0.x, x0.x, t);
+                    const e_grp x0 = load_x(gf);
+                    pair(w0.x, x0.q.x, x0.s.x, t);
                     acc = red_e<MODE>::clamped(t[0]);
                     t1 = t[1];
-                    fast8(w0, x0, w0.x, x0.x, 1);
+                    fast8(w0, x0, w0.x, x0, 1);
                 } else {
-                    uint4 x[PF];
+                    e_grp x[PF];
 #pragma unroll
                     for (int p = 0; p < PF; p++) x[p] = load_x(g + p);
-                    pair(wa[0].x, x[0].x, t);
+                    pair(wa[0].x, x[0].q.x, x[0].s.x, t);
                     t0 = t[0];
                     t1 = t[1];
 #pragma unroll
                     for (int p = 0; p < PF; p++)
                         if (g + p < full)
-                            fast8(wa[p], x[p], wa[p + 1 < PF ? p + 1 : p].x, x[p + 1 < PF ? p + 1 : p].x, 0);
+                            fast8(wa[p], x[p], wa[p + 1 < PF ? p + 1 : p].x, x[p + 1 < PF ? p + 1 : p], 0);
                 }
                 note();
                 redo = __any(mn < E::lo || mx > E::hi) != 0;
@@ -1920,7 +1943,7 @@ __device__ __forceinline__ void chain_e(const red_e<MODE> &R, const lfsr8_tab &L
 }
 
 // mme_chains for one chain per lane; head: its first weights
-template <int MODE, int PF, bool XL, bool HEAD>
+template <int MODE, int PF, bool XL, bool SPLIT, bool HEAD>
 __device__ __forceinline__ uint32_t mme_chain1(const mm_args16 &a, const dev_tables &T, const red_e<MODE> &R,
                                                const lfsr8_tab &L8, const uint16_t *xl, int64_t m, int64_t z,
                                                int64_t zw, int64_t zx, int64_t n0, const mm_head<PF> &head) {
@@ -1937,9 +1960,12 @@ __device__ __forceinline__ uint32_t mme_chain1(const mm_args16 &a, const dev_tab
     }
     auto load_w = [&](int g) { return *reinterpret_cast<const uint4 *>(ws + (int64_t)min(g, last) * wstride); };
     auto load_x = [&](int g) {   // (the offset through a vector register, as in mm16_chains)
-        int32_t off = min(g, last) * 8;
+        int32_t off = min(g, last) * (SPLIT ? 16 : 8);
         asm("" : "+v"(off));
-        return *reinterpret_cast<const uint4 *>(xs + off);
+        const uint4 *p = reinterpret_cast<const uint4 *>(xs + off);
+        e_grp r{p[0], uint4{}};
+        if constexpr (SPLIT) r.s = p[1];
+        return r;
     };
     uint4 wa[PF];
     if constexpr (HEAD) {
@@ -1949,7 +1975,7 @@ __device__ __forceinline__ uint32_t mme_chain1(const mm_args16 &a, const dev_tab
         mm16_wblock<PF>(a, m, zw, 1, wa);
     }
     int32_t acc = eform<MODE>::zero;
-    chain_e<MODE, PF>(R, L8, acc, st, 0, (int)a.K, HEAD ? head.w0 : load_w(0), wa,
+    chain_e<MODE, PF, SPLIT>(R, L8, acc, st, 0, (int)a.K, HEAD ? head.w0 : load_w(0), wa,
                       [&](uint4 (&w)[PF], int g) { mm16_wblock<PF>(a, m, zw, g, w); }, load_w, load_x);
     return red_e<MODE>::finish(acc) & 0xffffu;
 }
@@ -1962,14 +1988,15 @@ __device__ __forceinline__ uint32_t mme_chain1(const mm_args16 &a, const dev_tab
 // steps branch (lpvip's FP64 Gaussian log, the sign cases) and, measured,
 // run slower with part of the wave inactive (lpvip K 1536: 420 us with 16
 // lanes, 334 us with the same 16 chains on all 64, 313 us with 4 chains)
-// X32 (base and Monte, several columns): the activation rows are staged as the
-// one-word adders' words, 4 bytes each, where they fit LDS; RG groups of
-// k_block rows then share them, so that long rows leave room for enough waves
+// X32 (base and Monte, where they fit LDS): the activation rows take 4 bytes a
+// value, for several chains per lane the one-word adders' words, for one the
+// logs and signs of chain_e's SPLIT.  RG groups of k_block rows share the rows
+// of several columns, so that long rows leave room for enough waves
 // RB: rows of a column group (k_block, or 64 for column groups of one wave)
 template <int MODE, int NC, int PF, bool XL, int CG, int W = 64, bool X32 = false, int RG = 1, int RB = k_block>
 __global__ __launch_bounds__(RB *CG *RG) void k_mm16(mm_args16 a, dev_tables T) {
-    static_assert(!X32 || (is_e<MODE> && XL && NC > 1 && CG == 1), "word rows: base and Monte, several chains per lane");
-    static_assert(RG == 1 || X32, "row groups share word rows");
+    static_assert(!X32 || (is_e<MODE> && XL && CG == 1), "word rows: base and Monte");
+    static_assert(RG == 1 || (X32 && NC > 1), "row groups share word rows");
     static_assert(RB == k_block || (W == 64 && RG == 1), "whole waves");
     extern __shared__ __align__(16) char lds[];
     // a widened launch: the workgroups between the working ones leave at once
@@ -2098,7 +2125,13 @@ __global__ __launch_bounds__(RB *CG *RG) void k_mm16(mm_args16 a, dev_tables T) 
                         const int k = k0 + q * nt;
                         // (base and Monte: a column past N repeats the last
                         // one, whose sums stay in the fast form's range)
-                        if constexpr (X32) {
+                        if constexpr (X32 && NC == 1) {
+                            if (k < kp) {
+                                uint16_t *o = xl + (k >> 3) * 16 + (k & 7);
+                                o[0] = (uint16_t)(c[q] & k16_logmask);
+                                o[8] = (uint16_t)((c[q] >> 15) << (eform<is_e<MODE> ? MODE : LNSHIP_BASE>::sh - 2));
+                            }
+                        } else if constexpr (X32) {
                             // the word of a code, less the product's offset
                             if (k < kp)
                                 reinterpret_cast<int32_t *>(xl)[j * kp + k] =
@@ -2134,7 +2167,7 @@ __global__ __launch_bounds__(RB *CG *RG) void k_mm16(mm_args16 a, dev_tables T) 
     }
 
     uint32_t res[NC];
-    if constexpr (is_e<MODE> && NC == 1) res[0] = mme_chain1<MODE, PF, XL, head>(a, T, R, L8, xl, m, z, zw, zx, n0, hw);
+    if constexpr (is_e<MODE> && NC == 1) res[0] = mme_chain1<MODE, PF, XL, X32, head>(a, T, R, L8, xl, m, z, zw, zx, n0, hw);
     else if constexpr (is_e<MODE>) mme_chains<MODE, NC, PF, XL, X32>(a, T, R, L8, xl, m, z, zw, zx, n0, nc, res);
     else mm16_chains<MODE, NC, PF, XL, head>(a, T, R, xl, m, z, zw, zx, n0, nc, res, hw, slots);
     if (dup && lane % (64 / W) != 0) return;   // one lane of a chain stores
@@ -3487,7 +3520,7 @@ __device__ __forceinline__ uint32_t row_chain_e(const red_e<MODE> &R, const lfsr
     constexpr int PF = 4;
     const int gl = (k1 - 1) >> 3;
     auto load_w = [&](int g) { return *reinterpret_cast<const uint4 *>(w + (int64_t)min(g, gl) * gs); };
-    auto load_x = [&](int g) { return *reinterpret_cast<const uint4 *>(x + 8 * min(g, gl)); };
+    auto load_x = [&](int g) { return e_grp{*reinterpret_cast<const uint4 *>(x + 8 * min(g, gl)), uint4{}}; };
     auto block = [&](uint4 (&b)[PF], int g) {
 #pragma unroll
         for (int p = 0; p < PF; p++) b[p] = load_w(g + p);
@@ -3495,7 +3528,7 @@ __device__ __forceinline__ uint32_t row_chain_e(const red_e<MODE> &R, const lfsr
     uint4 wa[PF];
     block(wa, (k0 >> 3) + 1);
     int32_t acc = e_of<MODE>(a);
-    chain_e<MODE, PF>(R, L8, acc, st, k0, k1, load_w(k0 >> 3), wa, block, load_w, load_x);
+    chain_e<MODE, PF, false>(R, L8, acc, st, k0, k1, load_w(k0 >> 3), wa, block, load_w, load_x);
     return red_e<MODE>::finish(acc) & 0xffffu;
 }
 
@@ -4351,7 +4384,7 @@ static int launch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslices,
     // prefetch depth within 128 VGPRs at four waves per SIMD
     constexpr int PF = NC == 1 ? (CG * RB >= 4 * k_block ? 4 : 8) : NC == 2 ? 2 : (NC == 4 && CG < 4) ? 2 : 1;
     const int rows_lds = (XL ? (int)(NC * CG * m.kp * (X32 ? 4 : 2)) + k_xl_pad : 0) + (MODE == LNSHIP_LPVIP ? lp_slot_bytes(NC) : 0);
-    const bool no_tab = is_e<MODE> && NC == 1 && mm16_tab_bytes<MODE>() + rows_lds > k_lds_bytes - 1024;
+    const bool no_tab = is_e<MODE> && NC == 1 && !X32 && mm16_tab_bytes<MODE>() + rows_lds > k_lds_bytes - 1024;
     const int lds = (no_tab ? 0 : mm16_tab_bytes<MODE>()) + rows_lds;
     static_assert(PF * 16 <= k_xl_pad, "prefetch past the activation rows stays in the padding");
     // weight offsets within a block of PF groups are 32-bit
@@ -4429,6 +4462,17 @@ static int dispatch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslice
             case 8: return launch_mm16_x<MODE, 8, 1>(m, T, nslices, sh.xl, cus, st);
             case 4: return launch_mm16_x<MODE, 4, 1>(m, T, nslices, sh.xl, cus, st);
             default:
+                if constexpr (is_e<MODE>) {
+                    // the rows as logs and signs where they fit (one column,
+                    // per step: base 38 ns either way, Monte 49 at code width,
+                    // 46; K 1536, M 576, N 131: base 81.8 -> 75.1 us)
+                    if (sh.xl && mm16_tab_bytes<MODE>() + m.kp * 4 + k_xl_pad <= k_lds_bytes - 1024)
+                        switch (narrow_w(MODE, m.M * m.N * nslices, cus)) {
+                            case 16: return launch_mm16<MODE, 1, true, 1, 16, true>(m, T, nslices, cus, st);
+                            case 32: return launch_mm16<MODE, 1, true, 1, 32, true>(m, T, nslices, cus, st);
+                            default: return launch_mm16<MODE, 1, true, 1, 64, true>(m, T, nslices, cus, st);
+                        }
+                }
                 if (sh.xl) switch (narrow_w(MODE, m.M * m.N * nslices, cus)) {
                         case 4:
                             if constexpr (MODE == LNSHIP_LPVIP) return launch_mm16<MODE, 1, true, 1, 4>(m, T, nslices, cus, st);
