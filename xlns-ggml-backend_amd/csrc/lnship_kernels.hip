@@ -258,11 +258,17 @@ __device__ __forceinline__ cvt16_lds stage_cvt16(const uint16_t *cvt, uint16_t *
 // 2 xlns16 codes.  Bound by HBM: a thread converts runs of eight columns (one
 // 16-byte store for xlns16, two for xlns32), the lanes of a wave on eight
 // rows times eight runs, so that it reads 128 bytes or more of each row and
-// writes 128 bytes or more of each run; k_pack_c runs a thread, their loads
-// issued together.  Half 2048 x 8192 to xlns16: 34.9 -> 16.4 us (4.1 TB/s; one
-// element a thread, table gathers from global memory before).  vl, vs: the loads / the stores may be 16 bytes wide
-// (base and strides aligned); else element by element.
-constexpr int k_pack_rows = 32, k_pack_c = 4, k_pack_cols = 64 * k_pack_c;
+// writes 128 bytes or more of each run; for xlns16 four runs a thread, their
+// loads issued together.  Half 2048 x 8192 to xlns16: 34.9 -> 16.4 us (4.1
+// TB/s; one element a thread, table gathers from global memory before).
+// xlns32 is bound by its FP64 logarithms: one run a thread, so that a small
+// matrix still fills the chip (F32 3001 x 770: 23.3 us at four runs, 13.6 at
+// one; 8192 x 2048: 66.5 and 60.5, one element a thread 79).  vl, vs: the
+// loads / the stores may be 16 bytes wide (base and strides aligned); else
+// element by element.
+constexpr int k_pack_rows = 32;
+constexpr int k_pack_c(bool w32) { return w32 ? 1 : 4; }
+constexpr int k_pack_cols(bool w32) { return 64 * k_pack_c(w32); }
 template <int W32, int TY>
 __global__ __launch_bounds__(k_block) void k_pack(const void *__restrict__ src, int64_t src_ld, int64_t src_slice,
                                                   void *__restrict__ dst, int64_t rows, int64_t cols, int64_t kp,
@@ -275,15 +281,16 @@ __global__ __launch_bounds__(k_block) void k_pack(const void *__restrict__ src, 
         C = stage_cvt16(cvt, s_cvt);
         __syncthreads();
     }
-    const int64_t ctiles = (kp + k_pack_cols - 1) / k_pack_cols, rt = (int64_t)blockIdx.x / ctiles;
+    constexpr int NR = k_pack_c(W32);
+    const int64_t ctiles = (kp + k_pack_cols(W32) - 1) / k_pack_cols(W32), rt = (int64_t)blockIdx.x / ctiles;
     const int64_t r = rt * k_pack_rows + (threadIdx.x >> 3), z = blockIdx.y;
-    const int64_t g0 = ((int64_t)blockIdx.x - rt * ctiles) * (k_pack_cols / 8) + (threadIdx.x & 7);
+    const int64_t g0 = ((int64_t)blockIdx.x - rt * ctiles) * (8 * NR) + (threadIdx.x & 7);
     if (r >= rows) return;
     const src_t *s = reinterpret_cast<const src_t *>(src) + z * src_slice + r * src_ld;
     dst_t *d = reinterpret_cast<dst_t *>(dst) + z * rows * kp + r * 8;
-    src_t v[k_pack_c][8];
+    src_t v[NR][8];
 #pragma unroll
-    for (int q = 0; q < k_pack_c; q++) {
+    for (int q = 0; q < NR; q++) {
         const int64_t c0 = (g0 + 8 * q) * 8;
         if (vl && c0 + 8 <= cols) {
             union {
@@ -300,7 +307,7 @@ __global__ __launch_bounds__(k_block) void k_pack(const void *__restrict__ src, 
         }
     }
 #pragma unroll
-    for (int q = 0; q < k_pack_c; q++) {
+    for (int q = 0; q < NR; q++) {
         const int64_t g = g0 + 8 * q;
         if (g * 8 >= kp) continue;
         uint32_t c[8];
@@ -4230,7 +4237,7 @@ static int pack_common(int w32, const void *src, int src_is_f16, int64_t src_ld,
     if (src_is_f16 < 0 || src_is_f16 > (w32 ? 1 : 2)) return fail(LNSHIP_EINVAL, "pack: bad source type%s");
     if (K == 0 || M == 0 || nslices == 0) return 0;
     const int64_t kp = (K + 7) & ~(int64_t)7;
-    const int64_t tiles = ((M + k_pack_rows - 1) / k_pack_rows) * ((kp + k_pack_cols - 1) / k_pack_cols);
+    const int64_t tiles = ((M + k_pack_rows - 1) / k_pack_rows) * ((kp + k_pack_cols(w32) - 1) / k_pack_cols(w32));
     if (tiles > 0x7fffffff) return fail(LNSHIP_ERANGE, "pack: more than 2^31 tiles%s");
     dim3 grid((unsigned)tiles, (unsigned)nslices);
     const int64_t es = src_is_f16 == 0 ? 4 : 2;
