@@ -1223,6 +1223,7 @@ struct mm_args16 {
     // set by the launcher (base and Monte, one chain per lane): the rows leave
     // no room for the adder's table in LDS
     bool no_tab;
+    uint32_t y0;   // set by the launcher: the column block of the grid's first row
     // set by the launcher: the grid is 2^xcd_sh times wider than the work;
     // workgroup x works (as block x >> xcd_sh) iff x is a multiple of 2^xcd_sh
     uint32_t xcd_sh;
@@ -2011,7 +2012,7 @@ __global__ __launch_bounds__(RB *CG *RG) void k_mm16(mm_args16 a, dev_tables T) 
     // CG column groups of k_block lanes each share the staged tables: group
     // c takes columns [nw + c NC, nw + (c + 1) NC) of the same k_block rows
     const int cg = CG == 1 ? 0 : (int)(threadIdx.x / RB);
-    const int64_t nw = (int64_t)blockIdx.y * (NC * CG);
+    const int64_t nw = ((int64_t)blockIdx.y + a.y0) * (NC * CG);
     const int64_t n0 = nw + (int64_t)cg * NC;
     const int64_t z = blockIdx.z;
     const int64_t i12 = z % a.ne12, i13 = z / a.ne12;
@@ -4294,6 +4295,8 @@ static int mm16_nc(int mode, int64_t M, int64_t N, int64_t nslices, int64_t kp, 
     return 8;
 }
 
+constexpr int64_t k_grid_y = 65535;   // a launch's rows of workgroups
+
 struct mm16_shape {
     int nc, cg;   // columns per lane, column groups per workgroup
     bool xl;      // activations converted into LDS inside the kernel
@@ -4325,7 +4328,11 @@ static mm16_shape mm_shape_x32(int64_t M, int64_t N, int64_t nslices, int64_t kp
         // a group of 64 rows in place of one of 256 only where it needs no
         // scratch that the other did without
         if (rb == 64 && max_nc == 8 && best.xl && !xl) continue;
-        const int64_t wgs = (M + rb - 1) / rb * ((N + nc * cg - 1) / (nc * cg)) * nslices;
+        // nor where its grid or its threads pass a launch's limits and the
+        // other's (more columns a workgroup, or fewer threads a row) do not
+        const int64_t wg_m = (M + rb - 1) / rb, wg_n = (N + nc * cg - 1) / (nc * cg);
+        if (rb == 64 && (wg_n > k_grid_y || wg_m * cg * rb > 0xffffffff)) continue;
+        const int64_t wgs = wg_m * wg_n * nslices;
         const int64_t rounds = (wgs + std::max(cus, 1) - 1) / std::max(cus, 1);
         const int64_t step = waves == 1 ? (nc == 1 ? 166 : 148) : waves == 2 ? 103 : waves == 3 ? 91 : 85;
         const int64_t cost = rounds * waves * nc * step;
@@ -4400,14 +4407,21 @@ static int launch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslices,
     if (lds > 64 * 1024)
         if (int rc = set_lds(k_mm16<MODE, NC, PF, XL, CG, W, X32, RG, RB>, lds)) return rc;
     constexpr int rows = W < 64 ? k_block / 64 * W : RB * RG;   // rows per workgroup
-    dim3 grid((unsigned)((m.M + rows - 1) / rows), (unsigned)((m.N + NC * CG - 1) / (NC * CG)), (unsigned)nslices);
-    if (grid.x > 2147483647u || grid.y > 65535u) return fail(LNSHIP_ERANGE, "mul_mat: grid too large%s");
+    dim3 grid((unsigned)((m.M + rows - 1) / rows), 1, (unsigned)nslices);
+    if (grid.x > 2147483647u) return fail(LNSHIP_ERANGE, "mul_mat: grid too large%s");
+    const int64_t blocks = (m.N + NC * CG - 1) / (NC * CG);   // of columns
     mm_args16 mx = m;
     mx.no_tab = no_tab;
-    mx.xcd_sh = MODE == LNSHIP_SUM32 ? xcd_shift((uint64_t)grid.x * grid.y * grid.z, cus) : 0;
+    mx.xcd_sh = MODE == LNSHIP_SUM32 ? xcd_shift((uint64_t)grid.x * (uint64_t)blocks * grid.z, cus) : 0;
     grid.x <<= mx.xcd_sh;
-    hipLaunchKernelGGL((k_mm16<MODE, NC, PF, XL, CG, W, X32, RG, RB>), grid, dim3(RB * CG * RG), lds, st, mx, T);
-    LNSHIP_HIP(hipGetLastError());
+    // (more than one launch only where launch_mm16_x takes fewer columns a
+    // workgroup than the shape that dispatch_mm16 checked)
+    for (int64_t y0 = 0; y0 < blocks; y0 += k_grid_y) {
+        mx.y0 = (uint32_t)y0;
+        grid.y = (unsigned)std::min(blocks - y0, k_grid_y);
+        hipLaunchKernelGGL((k_mm16<MODE, NC, PF, XL, CG, W, X32, RG, RB>), grid, dim3(RB * CG * RG), lds, st, mx, T);
+        LNSHIP_HIP(hipGetLastError());
+    }
     return 0;
 }
 
@@ -4431,8 +4445,11 @@ static int launch_mm16_x(const mm_args16 &m, const dev_tables &T, int64_t nslice
         }
     }
     if constexpr (NC > 1 && MODE != LNSHIP_SUM32) {
-        // rows that fill the LDS beside what several chains take (one row
-        // per workgroup then)
+        // Rows that fill the LDS beside what several chains take: one row per
+        // workgroup.  (Four rows, which would fit beside the tables of eight,
+        // leave a CU one workgroup of four waves: M 2048, N 512, Monte K 8192
+        // 6.28 ms against 3.40, base K 9704 4.61 against 2.88, lpvip K 9400
+        // 10.8 against 8.6.)
         if (xl && mm16_tab_bytes<MODE>() + (MODE == LNSHIP_LPVIP ? lp_slot_bytes(NC) : 0) + (int64_t)NC * m.kp * 2 + k_xl_pad > k_lds_bytes - 1024)
             return launch_mm16<MODE, 1, true, 1>(m, T, nslices, cus, st);
     }
@@ -4443,6 +4460,7 @@ static int launch_mm16_x(const mm_args16 &m, const dev_tables &T, int64_t nslice
 template <int MODE>
 static int dispatch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslices, const mm16_shape &sh,
                          int cus, hipStream_t st) {
+    if (m.N > k_grid_y * sh.nc * sh.cg) return fail(LNSHIP_ERANGE, "mul_mat: grid too large%s");
     if constexpr (MODE == LNSHIP_SUM32) {
         // column groups: more waves per SIMD where the tables allow one
         // workgroup per CU
