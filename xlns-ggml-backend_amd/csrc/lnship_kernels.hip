@@ -255,86 +255,89 @@ __device__ __forceinline__ cvt16_lds stage_cvt16(const uint16_t *cvt, uint16_t *
 
 // rows x cols row-major -> k8-interleaved (k = col, m = row), one slice per
 // blockIdx.y; padding columns (cols..Kp) get code 0.  TY: 0 F32, 1 IEEE half,
-// 2 xlns16 codes.  Bound by HBM: a thread converts runs of eight columns (one
-// 16-byte store for xlns16, two for xlns32), the lanes of a wave on eight
-// rows times eight runs, so that it reads 128 bytes or more of each row and
-// writes 128 bytes or more of each run; for xlns16 four runs a thread, their
-// loads issued together.  Half 2048 x 8192 to xlns16: 34.9 -> 16.4 us (4.1
-// TB/s; one element a thread, table gathers from global memory before).
-// xlns32 is bound by its FP64 logarithms: one run a thread, so that a small
-// matrix still fills the chip (F32 3001 x 770: 23.3 us at four runs, 13.6 at
-// one; 8192 x 2048: 66.5 and 60.5, one element a thread 79).  vl, vs: the
-// loads / the stores may be 16 bytes wide (base and strides aligned); else
-// element by element.
-constexpr int k_pack_rows = 32;
-constexpr int k_pack_c(bool w32) { return w32 ? 1 : 4; }
-constexpr int k_pack_cols(bool w32) { return 64 * k_pack_c(w32); }
-template <int W32, int TY>
+// 2 xlns16 codes.  Bound by HBM (xlns32: by its FP64 logarithms): a thread
+// converts NR runs of RN neighbouring columns, in 16-byte loads and stores
+// where those are aligned, the workgroup's threads on p.lanes neighbouring
+// runs of p.rows rows.  Runs of one column are for matrices of few workgroups,
+// bound by latency (xlns16: without the table's staging).  Half 2048 x 8192 to
+// xlns16: 15.5 us (4.3 TB/s; one element a thread 34.9).  The shapes and what
+// they measured: choose_pack.
+struct pack_shape {
+    int lanes, rows;   // neighbouring runs of a row, rows of a tile
+    uint32_t recip;    // ceil(2^16 / lanes): t / lanes = t recip >> 16 for t < k_block
+    int64_t ctiles, tiles;
+    int run, nr;
+    bool vl, vs;       // the loads / the stores are 16 (or 8) bytes wide
+};
+template <int W32, int TY, int RN, int NR>
 __global__ __launch_bounds__(k_block) void k_pack(const void *__restrict__ src, int64_t src_ld, int64_t src_slice,
                                                   void *__restrict__ dst, int64_t rows, int64_t cols, int64_t kp,
-                                                  bool vl, bool vs, const uint16_t *__restrict__ cvt) {
+                                                  pack_shape p, int64_t t0, const uint16_t *__restrict__ cvt) {
     using src_t = typename std::conditional<TY == 0, uint32_t, uint16_t>::type;
     using dst_t = typename std::conditional<W32 != 0, uint32_t, uint16_t>::type;
+    constexpr int bytes = RN * (int)sizeof(src_t);
+    using vec_t = typename std::conditional<bytes >= 16, uint4, typename std::conditional<bytes == 8, uint2, src_t>::type>::type;
     __shared__ uint16_t s_cvt[k_cvt_lds];
+    const int64_t z = blockIdx.y, t = t0 + (int64_t)blockIdx.x, rt = t / p.ctiles;
+    const int tr = (int)(threadIdx.x * p.recip >> 16), tc = (int)threadIdx.x - tr * p.lanes;
+    const int64_t r = rt * p.rows + tr;
+    const int64_t g0 = (t - rt * p.ctiles) * (NR * p.lanes) + tc;
     cvt16_lds C{};
-    if constexpr (!W32 && TY != 2) {
+    if constexpr (!W32 && TY != 2 && RN > 1) {
         C = stage_cvt16(cvt, s_cvt);
         __syncthreads();
     }
-    constexpr int NR = k_pack_c(W32);
-    const int64_t ctiles = (kp + k_pack_cols(W32) - 1) / k_pack_cols(W32), rt = (int64_t)blockIdx.x / ctiles;
-    const int64_t r = rt * k_pack_rows + (threadIdx.x >> 3), z = blockIdx.y;
-    const int64_t g0 = ((int64_t)blockIdx.x - rt * ctiles) * (8 * NR) + (threadIdx.x & 7);
-    if (r >= rows) return;
+    if (tr >= p.rows || r >= rows) return;
     const src_t *s = reinterpret_cast<const src_t *>(src) + z * src_slice + r * src_ld;
     dst_t *d = reinterpret_cast<dst_t *>(dst) + z * rows * kp + r * 8;
-    src_t v[NR][8];
+    src_t v[NR][RN];
 #pragma unroll
     for (int q = 0; q < NR; q++) {
-        const int64_t c0 = (g0 + 8 * q) * 8;
-        if (vl && c0 + 8 <= cols) {
+        const int64_t c0 = (g0 + (int64_t)q * p.lanes) * RN;
+        if (p.vl && c0 + RN <= cols) {
             union {
-                uint4 w[sizeof(src_t) / 2];
-                src_t e[8];
+                vec_t w[bytes / sizeof(vec_t)];
+                src_t e[RN];
             } u;
 #pragma unroll
-            for (int i = 0; i < (int)sizeof(src_t) / 2; i++) u.w[i] = reinterpret_cast<const uint4 *>(s + c0)[i];
+            for (int i = 0; i < bytes / (int)sizeof(vec_t); i++) u.w[i] = reinterpret_cast<const vec_t *>(s + c0)[i];
 #pragma unroll
-            for (int i = 0; i < 8; i++) v[q][i] = u.e[i];
+            for (int i = 0; i < RN; i++) v[q][i] = u.e[i];
         } else {
 #pragma unroll
-            for (int i = 0; i < 8; i++) v[q][i] = c0 + i < cols ? s[c0 + i] : (src_t)0;
+            for (int i = 0; i < RN; i++) v[q][i] = c0 + i < cols ? s[c0 + i] : (src_t)0;
         }
     }
 #pragma unroll
     for (int q = 0; q < NR; q++) {
-        const int64_t g = g0 + 8 * q;
-        if (g * 8 >= kp) continue;
-        uint32_t c[8];
+        const int64_t c0 = (g0 + (int64_t)q * p.lanes) * RN;
+        if (c0 >= kp) continue;
+        uint32_t c[RN];
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
+        for (int i = 0; i < RN; i++) {
             if constexpr (TY == 2) {
                 c[i] = v[q][i];
             } else {
                 float f;
                 if constexpr (TY == 1) f = __half2float(__ushort_as_half(v[q][i]));
                 else f = __uint_as_float(v[q][i]);
-                c[i] = W32 ? x32_from_f32(f) : C(f);
+                c[i] = W32 ? x32_from_f32(f) : RN > 1 ? C(f) : x16_from_f32(cvt, f);
             }
-            if (g * 8 + i >= cols) c[i] = 0u;
+            if (c0 + i >= cols) c[i] = 0u;
         }
-        dst_t *o = d + g * rows * 8;
-        if (vs) {
+        dst_t *o = d + (c0 >> 3) * rows * 8 + (c0 & 7);
+        if (RN > 1 && p.vs) {
             if constexpr (W32) {
-                reinterpret_cast<uint4 *>(o)[0] = make_uint4(c[0], c[1], c[2], c[3]);
-                reinterpret_cast<uint4 *>(o)[1] = make_uint4(c[4], c[5], c[6], c[7]);
+#pragma unroll
+                for (int i = 0; i + 3 < RN; i += 4)
+                    reinterpret_cast<uint4 *>(o)[i / 4] = make_uint4(c[i], c[i + 1], c[i + 2], c[i + 3]);
             } else {
                 *reinterpret_cast<uint4 *>(o) = make_uint4(c[0] | c[1] << 16, c[2] | c[3] << 16, c[4] | c[5] << 16,
                                                            c[6] | c[7] << 16);
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < 8; i++) o[i] = (dst_t)c[i];
+            for (int i = 0; i < RN; i++) o[i] = (dst_t)c[i];
         }
     }
 }
@@ -4229,6 +4232,48 @@ static int set_lds(K kernel, int bytes) {
     return 0;
 }
 
+// Lanes on neighbouring runs of a row: 64 columns of it, so that a wave reads
+// 128 bytes or more of each row and writes 128 bytes or more of each run; all
+// of a row's runs where those are fewer (K 8, M 1e6, half: 58.1 us with idle
+// lanes for the rest of eight, 8.4 so), and more where the rows are fewer than
+// a tile's (K 1e6, M 1, F32: 9.2 and 3.1 us).
+// xlns16: one run of eight a thread; four, whose loads go out together, share
+// the conversion table's staging, which pays for large sources that load
+// element by element (F32 577 x 49152: 51.0 us, one run 54.3; 577 x 3000: 10.3
+// and 5.7).  Tiny matrices: one column a thread, its code from global memory
+// (256 x 256: 2.6 us in runs, 2.2 so).
+// xlns32: runs of eight where the tiles fill the chip several times (2048 x
+// 8192: 55.0 us, in runs of four 57.3), else of four (576 x 1536: 6.8 and 6.2),
+// of one where those do not fill it (256 x 256: 3.1 in runs of four, 2.2 so).
+static pack_shape choose_pack(int w32, const void *src, int type, int64_t src_ld, int64_t src_slice, const void *dst,
+                              int64_t kp, int64_t M, int64_t nslices) {
+    const int64_t es = type == 0 ? 4 : 2;
+    pack_shape p{};
+    p.vl = (uintptr_t)src % 16 == 0 && src_ld * es % 16 == 0 && (nslices == 1 || src_slice * es % 16 == 0);
+    p.vs = (uintptr_t)dst % 16 == 0;
+    auto shape = [&](int run, int nr) {
+        const int64_t most = std::max<int64_t>(64 / run, M < 32 ? k_block / M : 0);   // lanes of a row
+        const int64_t runs = kp / run, tiles = (runs + most - 1) / most;
+        p.run = run;
+        p.nr = nr;
+        p.lanes = (int)((runs + tiles - 1) / tiles);
+        p.rows = k_block / p.lanes;
+        p.recip = (uint32_t)((65536 + p.lanes - 1) / p.lanes);
+        p.ctiles = (runs + (int64_t)nr * p.lanes - 1) / ((int64_t)nr * p.lanes);
+        p.tiles = (M + p.rows - 1) / p.rows * p.ctiles;
+    };
+    if (w32) {
+        shape(8, 1);
+        if (p.tiles * nslices < 2048) shape(4, 1);
+        if (p.run == 4 && p.tiles * nslices < 300) shape(1, 1);
+    } else {
+        shape(8, 4);
+        if (p.vl || type == 2 || p.tiles * nslices < 4096) shape(8, 1);
+        if (type != 2 && p.tiles * nslices < 100) shape(1, 1);
+    }
+    return p;
+}
+
 static int pack_common(int w32, const void *src, int src_is_f16, int64_t src_ld, int64_t src_slice, void *dst,
                        int64_t K, int64_t M, int64_t nslices, void *stream) {
     device_state *s = state();
@@ -4238,18 +4283,27 @@ static int pack_common(int w32, const void *src, int src_is_f16, int64_t src_ld,
     if (src_is_f16 < 0 || src_is_f16 > (w32 ? 1 : 2)) return fail(LNSHIP_EINVAL, "pack: bad source type%s");
     if (K == 0 || M == 0 || nslices == 0) return 0;
     const int64_t kp = (K + 7) & ~(int64_t)7;
-    const int64_t tiles = ((M + k_pack_rows - 1) / k_pack_rows) * ((kp + k_pack_cols(w32) - 1) / k_pack_cols(w32));
-    if (tiles > 0x7fffffff) return fail(LNSHIP_ERANGE, "pack: more than 2^31 tiles%s");
-    dim3 grid((unsigned)tiles, (unsigned)nslices);
-    const int64_t es = src_is_f16 == 0 ? 4 : 2;
-    const bool vl = (uintptr_t)src % 16 == 0 && src_ld * es % 16 == 0 && (nslices == 1 || src_slice * es % 16 == 0);
-    const bool vs = (uintptr_t)dst % 16 == 0;
+    const pack_shape p = choose_pack(w32, src, src_is_f16, src_ld, src_slice, dst, kp, M, nslices);
     auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(k_block), 0, (hipStream_t)stream, src, src_ld, src_slice, dst, M, K, kp,
-                           vl, vs, s->T.cvt16);
+        // (a launch takes fewer than 2^32 threads)
+        constexpr int64_t most = (int64_t)1 << 23;
+        for (int64_t t0 = 0; t0 < p.tiles; t0 += most)
+            hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(p.tiles - t0, most), (unsigned)nslices), dim3(k_block), 0,
+                               (hipStream_t)stream, src, src_ld, src_slice, dst, M, K, kp, p, t0, s->T.cvt16);
     };
-    if (w32) src_is_f16 ? go(k_pack<1, 1>) : go(k_pack<1, 0>);
-    else src_is_f16 == 2 ? go(k_pack<0, 2>) : src_is_f16 ? go(k_pack<0, 1>) : go(k_pack<0, 0>);
+    auto go32 = [&](auto ty) {
+        constexpr int TY = decltype(ty)::value;
+        p.run == 8 ? go(k_pack<1, TY, 8, 1>) : p.run == 4 ? go(k_pack<1, TY, 4, 1>) : go(k_pack<1, TY, 1, 1>);
+    };
+    auto go16 = [&](auto ty) {
+        constexpr int TY = decltype(ty)::value;
+        p.nr == 4 ? go(k_pack<0, TY, 8, 4>) : p.run == 8 ? go(k_pack<0, TY, 8, 1>) : go(k_pack<0, TY, 1, 1>);
+    };
+    using f32 = std::integral_constant<int, 0>;
+    using f16 = std::integral_constant<int, 1>;
+    if (w32) src_is_f16 ? go32(f16{}) : go32(f32{});
+    else if (src_is_f16 == 2) go(k_pack<0, 2, 8, 1>);
+    else src_is_f16 ? go16(f16{}) : go16(f32{});
     LNSHIP_HIP(hipGetLastError());
     return 0;
 }
