@@ -2924,14 +2924,16 @@ __device__ __forceinline__ const float *mask_row(const sm_args &a, int64_t row) 
 // The element passes are bound by their table reads and by the wavefronts in
 // flight, the sums by their chains.  Up to 16 waves per workgroup, 2^gs lanes
 // per row (no division to place an element, the row's maximum and last nonzero
-// exp by lane exchanges), the conversions and (GL) the Gaussian logs from LDS,
+// exp by lane exchanges; WIDE: several waves of lanes, for rows so few that a
+// wave each would leave waves idle: one row of 8192, base 343 -> 306 us, sum32
+// 428 -> 393), the conversions and (GL) the Gaussian logs from LDS,
 // the mask's addition only where a mask value is neither 0 nor -inf.  32 heads
 // of 512 x 512 under a causal mask: 114 -> 56 us (base), 203 -> 113 (sum32).
 template <int MODE, bool GL>
 constexpr int sm16_tables() {
     return ((row_tables_bytes<MODE>() + 15) & ~15) + (GL ? (2 * k16_gauss_n * 2 + 15) & ~15 : 0);
 }
-template <int MODE, bool GL>
+template <int MODE, bool GL, bool WIDE>
 __global__ __launch_bounds__(4 * k_block) void k_softmax16(sm_args a, dev_tables T) {
     extern __shared__ __align__(16) char lds[];
     const auto R = stage_rows<MODE>(T, lds);
@@ -2952,7 +2954,13 @@ __global__ __launch_bounds__(4 * k_block) void k_softmax16(sm_args a, dev_tables
     const int nr = (int)min<int64_t>(a.rb, a.ne1 * a.ne2 * a.ne3 - r0);
     const int n = (int)a.n;        // a row fits in LDS, so 32-bit counts suffice
     const int rs = (n + 7) & ~7;   // LDS rows 16-byte aligned
-    if ((int)threadIdx.x < nr) s_mrow[threadIdx.x] = a.mask ? mask_row(a, r0 + threadIdx.x) : nullptr;
+    if ((int)threadIdx.x < nr) {
+        s_mrow[threadIdx.x] = a.mask ? mask_row(a, r0 + threadIdx.x) : nullptr;
+        if constexpr (WIDE) {
+            s_tot[threadIdx.x] = (uint32_t)x16_canon(0xffffu);
+            s_last[threadIdx.x] = 0;
+        }
+    }
     __syncthreads();
     const uint32_t sc = x16_from_f32(T.cvt16, a.scale);
     const bool has_mask = a.mask != nullptr;
@@ -2961,9 +2969,10 @@ __global__ __launch_bounds__(4 * k_block) void k_softmax16(sm_args a, dev_tables
     // for.  Past the end a lane loads the last element again.
     constexpr int B = 4;   // (8 keeps more waves out than it hides: C5's rows 78 us at 8, 56 at 4)
     const int G = 1 << a.gs, i0 = (int)threadIdx.x & (G - 1), rstep = (int)blockDim.x >> a.gs;
-    for (int r = (int)threadIdx.x >> a.gs; r < nr; r += rstep) {
+    // the row's soft_max inputs into LDS; the largest, canonical, of the
+    // row's lanes in the wave
+    auto inputs = [&](int r, uint16_t *row) __attribute__((always_inline)) {
         const float *src = a.src + (r0 + r) * a.n, *mrow = s_mrow[r];
-        uint16_t *row = c + r * rs;
         int32_t cm = x16_canon(0xffffu);
         for (int e0 = i0; e0 < n; e0 += B * G) {
             float f[B], mf[B];
@@ -3006,9 +3015,13 @@ __global__ __launch_bounds__(4 * k_block) void k_softmax16(sm_args a, dev_tables
                 if (e0 + q * G < n) row[e0 + q * G] = (uint16_t)w[q];
             }
         }
-        for (int o = G >> 1; o > 0; o >>= 1) cm = max(cm, __shfl_xor(cm, o));
+        for (int o = (WIDE ? 64 : G) >> 1; o > 0; o >>= 1) cm = max(cm, __shfl_xor(cm, o));
+        return cm;
+    };
+    // the exps in place (a lane reads back its own elements); the last
+    // nonzero one of the row's lanes in the wave
+    auto exps = [&](uint16_t *row, int32_t cm) __attribute__((always_inline)) {
         const uint32_t mx = (uint32_t)(uint16_t)(cm < 0 ? (cm ^ 0x7fff) : cm) ^ k16_sign;
-        // the exps in place (a lane reads back its own elements)
         int last = 0;
         for (int e0 = i0; e0 < n; e0 += B * G) {
             uint32_t x[B];
@@ -3025,8 +3038,28 @@ __global__ __launch_bounds__(4 * k_block) void k_softmax16(sm_args a, dev_tables
                     if (x[q] & k16_logmask) last = e0 + q * G;
                 }
         }
-        for (int o = G >> 1; o > 0; o >>= 1) last = max(last, __shfl_xor(last, o));
-        if (i0 == 0) s_last[r] = last;
+        for (int o = (WIDE ? 64 : G) >> 1; o > 0; o >>= 1) last = max(last, __shfl_xor(last, o));
+        return last;
+    };
+    if constexpr (!WIDE) {
+        for (int r = (int)threadIdx.x >> a.gs; r < nr; r += rstep) {
+            uint16_t *row = c + r * rs;
+            const int last = exps(row, inputs(r, row));
+            if (i0 == 0) s_last[r] = last;
+        }
+    } else {
+        // a row on several waves: their maxima meet in s_max (s_tot's place,
+        // until the sums), then their last nonzero exps
+        int32_t *s_max = reinterpret_cast<int32_t *>(s_tot);
+        for (int r = (int)threadIdx.x >> a.gs; r < nr; r += rstep) {
+            const int32_t cm = inputs(r, c + r * rs);
+            if ((i0 & 63) == 0) atomicMax(&s_max[r], cm);
+        }
+        __syncthreads();
+        for (int r = (int)threadIdx.x >> a.gs; r < nr; r += rstep) {
+            const int last = exps(c + r * rs, s_max[r]);
+            if ((i0 & 63) == 0) atomicMax(&s_last[r], last);
+        }
     }
     __syncthreads();
     // (all 64 lanes, as in k_rms16)
@@ -4216,12 +4249,13 @@ static int64_t row_limit() { return max_row(MODE == LNSHIP_SUM32 ? k_lds_pos32 :
 // The most rows LDS holds decide how many rounds of blocks the GPU needs;
 // within that many rounds the rows are spread over every block slot, so that
 // no block carries more rows (longer element passes) than it must.
-static int rows_per_block(int tab_bytes, int64_t ncols, int elem_bytes, int64_t nrows, int cus) {
+// most: the workgroups a CU runs at once, LDS aside.
+static int rows_per_block(int tab_bytes, int64_t ncols, int elem_bytes, int64_t nrows, int cus, int64_t most = INT64_MAX) {
     const int64_t tabs = (tab_bytes + 15) & ~15;
     const int64_t row = std::max<int64_t>(1, ncols * elem_bytes);
     const int64_t rb_max = std::min<int64_t>(64, (k_lds_bytes - tabs - k_lds_static) / row);
     if (rb_max < 1 || nrows < 1) return (int)rb_max;
-    const int64_t slots = (int64_t)std::max(cus, 1) * std::max<int64_t>(1, k_lds_bytes / (tabs + rb_max * row));
+    const int64_t slots = (int64_t)std::max(cus, 1) * std::max<int64_t>(1, std::min(most, k_lds_bytes / (tabs + rb_max * row)));
     const int64_t rounds = (nrows + rb_max * slots - 1) / (rb_max * slots);
     return (int)std::min<int64_t>(rb_max, (nrows + rounds * slots - 1) / (rounds * slots));
 }
@@ -4669,13 +4703,17 @@ static int launch_sm16(sm_args &m, int64_t nrows, const dev_tables &T, int cus, 
     auto rounds = [&](int rb, int tab) {
         return rb < 1 ? INT64_MAX : (nrows + (int64_t)rb * cus - 1) / ((int64_t)rb * cus * std::max<int64_t>(1, k_lds_bytes / (tab + rb * rs * 2)));
     };
-    const int rb_g = rows_per_block(sm16_tables<MODE, true>(), rs, 2, nrows, cus);
-    const int rb_n = rows_per_block(sm16_tables<MODE, false>(), rs, 2, nrows, cus);
+    // (a CU runs 32 waves)
+    const int rb_g = rows_per_block(sm16_tables<MODE, true>(), rs, 2, nrows, cus, 8);
+    const int rb_n = rows_per_block(sm16_tables<MODE, false>(), rs, 2, nrows, cus, 8);
     const bool gl = rb_g >= 1 && rounds(rb_g, sm16_tables<MODE, true>()) <= rounds(rb_n, sm16_tables<MODE, false>());
     m.rb = gl ? rb_g : rb_n;
     if (m.rb < 1) return fail(LNSHIP_ERANGE, "soft_max: row too long for LDS%s");
     m.gs = 6;
-    while (m.gs > 3 && m.n <= (int64_t)1 << (m.gs - 1)) m.gs--;
+    // (a lane takes batches of four: fewer lanes a row where the rows are many;
+    // 20000 rows of 33, sum32: 30.2 us on 64 lanes a row, 18.9 on 16)
+    const int64_t one = nrows >= (int64_t)cus * 16 ? 4 : 1;
+    while (m.gs > (one > 1 ? 2 : 3) && m.n <= one << (m.gs - 1)) m.gs--;
     const int tab = gl ? sm16_tables<MODE, true>() : sm16_tables<MODE, false>();
     // a row for each group of lanes of a four-wave workgroup where there are
     // that many (2048 rows of 64: 17.5 us at one row a workgroup, 11.1 so)
@@ -4684,17 +4722,22 @@ static int launch_sm16(sm_args &m, int64_t nrows, const dev_tables &T, int cus, 
     // about sixteen waves on a CU, over the workgroups that share it
     const int64_t wgs = (nrows + m.rb - 1) / m.rb;
     const int64_t share = std::min<int64_t>(std::max<int64_t>(1, k_lds_bytes / (tab + m.rb * rs * 2)), (wgs + cus - 1) / std::max(cus, 1));
-    const int64_t waves = std::max<int64_t>(4, std::min<int64_t>(16 / std::max<int64_t>(share, 1), ((m.rb << m.gs) + 63) / 64));
-    const int threads = (int)waves * 64;
-    const int lds = (gl ? sm16_tables<MODE, true>() : sm16_tables<MODE, false>()) + (int)(m.rb * rs * 2);
-    const dim3 grid((unsigned)((nrows + m.rb - 1) / m.rb));
-    if (gl) {
-        if (int rc = set_lds(k_softmax16<MODE, true>, lds)) return rc;
-        hipLaunchKernelGGL((k_softmax16<MODE, true>), grid, dim3(threads), lds, st, m, T);
-    } else {
-        if (int rc = set_lds(k_softmax16<MODE, false>, lds)) return rc;
-        hipLaunchKernelGGL((k_softmax16<MODE, false>), grid, dim3(threads), lds, st, m, T);
-    }
+    const int64_t most = std::max<int64_t>(4, 16 / std::max<int64_t>(share, 1));
+    // several waves a row where the rows leave them idle and each has two batches
+    while (m.gs >= 6 && ((int64_t)m.rb << (m.gs + 1)) <= most * 64 && m.n >= (int64_t)8 << m.gs) m.gs++;
+    const int64_t waves = std::max<int64_t>(4, std::min<int64_t>(most, (((int64_t)m.rb << m.gs) + 63) / 64));
+    // (a launch takes fewer than 2^32 threads)
+    const int threads = (int)(wgs * waves < (int64_t)1 << 26 ? waves * 64 : k_block);
+    const int lds = tab + (int)(m.rb * rs * 2);
+    const dim3 grid((unsigned)wgs);
+    auto go = [&](auto kernel) {
+        if (int rc = set_lds(kernel, lds)) return rc;
+        hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, st, m, T);
+        return 0;
+    };
+    if (int rc = m.gs > 6 ? gl ? go(k_softmax16<MODE, true, true>) : go(k_softmax16<MODE, false, true>)
+                          : gl ? go(k_softmax16<MODE, true, false>) : go(k_softmax16<MODE, false, false>))
+        return rc;
     LNSHIP_HIP(hipGetLastError());
     return 0;
 }
