@@ -399,6 +399,11 @@ typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pk_sub_sat_u16(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
 }
+__device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
+    uint32_t r;
+    asm("v_pk_max_u16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
 __device__ __forceinline__ uint32_t pk_min_u16(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
 }
@@ -921,7 +926,10 @@ __device__ __forceinline__ void stage_copy(int4 *dst, const int4 *__restrict__ s
 // either way; exact cancellation leaves a negative word, which every later
 // term exceeds from beyond `far`.  The chains run in blocks: a block records
 // the least and the largest M of its steps, and one that leaves the range is
-// run again by the exact form (xstep), which clamps.
+// run again by the exact form (xstep1, xread and xsum), which clamps, and so do
+// the next blocks (k_hold): data with runs of zeros leaves it again and again
+// (K 8192, M 2048, one column of zeros: base 424 us with the clamping adder, 382
+// so; half of the activations zero: 425 and 359).
 //
 // Measured on MI355X against the clamping adder with log and sign apart: a
 // single chain's step 51 -> 38 ns (base) and 65 -> 46 ns (Monte); the product
@@ -962,6 +970,8 @@ __device__ __forceinline__ void e_words(uint32_t lm, uint32_t sg, uint32_t k_em,
     t[0] = (int32_t)bfi1(k_em, lm << eform<MODE>::sh, sg);
     t[1] = (int32_t)bfi1(k_em, lm >> (16 - eform<MODE>::sh), sg >> 16);
 }
+// the first part's log fields clamped as xlns16_mul clamps a product's log
+__device__ __forceinline__ uint32_t e_clamp(uint32_t lm) { return pk_min_u16(pk_max_u16(lm, 0x40004000u), 0xbfffbfffu); }
 // the first part with the activations' half of it staged: their logs, and
 // their signs at u's place
 template <int MODE>
@@ -983,29 +993,27 @@ __device__ __forceinline__ e_masks e_mask_regs() {
 }
 typedef const int16_t __attribute__((address_space(3))) *lds_i16_t;
 typedef const uint16_t __attribute__((address_space(3))) *lds_u16_t;
-template <int MODE, bool POS = false>
+// TIGHT: for launches whose rows leave no room for all the tables: base's is the
+// narrow one, at tb with four bytes a distance (its entries' addresses take
+// four more instructions a step); Monte's draws come step by step
+template <int MODE, bool POS = false, bool TIGHT = false>
 struct red_e {
     using E = eform<MODE, POS>;
     uint32_t tb, cap;   // LDS byte addresses of the table and of its last entry
     uint32_t scale;     // 2^sh in a register the compiler cannot see into
-    // non-null: the table in global memory, for launches whose rows leave no
-    // room for it in LDS (tb is 0); only exact steps run then
-    const char *g;
     // the address of the entry for words x and y: their distance, the table's
     // base added by the same instruction, capped
     __device__ __forceinline__ uint32_t at(int32_t x, int32_t y) const {
         return min(sad_u32((uint32_t)x, (uint32_t)y, tb), cap);
     }
     __device__ __forceinline__ int32_t entry(uint32_t va) const {
+        if constexpr (TIGHT && !E::monte && !POS) {
+            const uint32_t v = va - tb;
+            va = tb + ((v + E::u) >> E::sh << 2) + (v & E::u);
+        }
         if constexpr (E::monte && !POS) return lds_ld(va);
         else if constexpr (E::monte) return *(lds_u16_t)(uintptr_t)va;
         else return *(lds_i16_t)(uintptr_t)va;
-    }
-    __device__ __forceinline__ int32_t entry_any(uint32_t va) const {
-        if (__builtin_expect(g == nullptr, 1)) return entry(va);
-        if constexpr (E::monte && !POS) return *reinterpret_cast<const int32_t *>(g + va);
-        else if constexpr (E::monte) return *reinterpret_cast<const uint16_t *>(g + va);
-        else return *reinterpret_cast<const int16_t *>(g + va);
     }
     // the sum: the larger word M and the adjustment of entry en at address va;
     // r: Monte's draw, the top 6 bits of the LFSR state.  Monte's entries are
@@ -1045,20 +1053,67 @@ struct red_e {
         else a = sum(M, en, dr);
         return M;
     }
+    static __device__ __forceinline__ int32_t med3(int32_t x, int32_t lo, int32_t hi) {
+        int32_t r;
+        asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(lo), "v"(hi));
+        return r;
+    }
+    // the words of the ends of the log field with the sum's sign, the larger
+    // operand's (exact cancellation, whose sum lies below: +0)
+    __device__ __forceinline__ void bounds(uint32_t va, int32_t M, int32_t &lo, int32_t &hi) const {
+        const int32_t s = M & (int32_t)E::u;
+        hi = (E::hi - (int32_t)E::u) | s;
+        lo = E::zero | s;
+        if constexpr (!POS) lo = va == tb + E::u ? E::zero : lo;
+    }
+    // step1 for any words t within the log field (e_clamp) and any a: the
+    // sum's clamps, which keep its sign (exact cancellation: +0), as one
+    // v_med3 between bounds formed in the round trip.  A step (K 8192, M 2048,
+    // every activation zero): base 47 ns, Monte 56, against 39 and 46 of step1
+    // and 52 and 66 of the adder with log and sign apart.
+    template <class F>
+    __device__ __forceinline__ void xstep1(int32_t &a, int32_t t, uint32_t r, F &&shadow) const {
+        uint32_t va;
+        asm("v_sad_u32 %0, %1, %2, %3\n\tv_min_u32 %0, %0, %4" : "=&v"(va) : "v"(a), "v"(t), "v"(tb), "v"(cap));
+        const int32_t en = entry(va);
+        __builtin_amdgcn_sched_barrier(0);
+        const int32_t M = max(a, t);
+        const uint32_t dr = E::monte ? draw(va, r) : 0u;
+        int32_t lo, hi;
+        bounds(va, M, lo, hi);
+        shadow();
+        asm volatile("" ::"v"(M), "v"(dr), "v"(lo), "v"(hi));
+        __builtin_amdgcn_sched_barrier(0);
+        int32_t x;
+        if constexpr (E::monte) x = __mul24((int32_t)(dr + (uint32_t)en) >> 6, (int32_t)scale) + M;
+        else x = sum(M, en, dr);
+        a = med3(x, lo, hi);
+    }
     // a word as the reference's clamps leave it: the log within its field,
     // the sign kept
     static __device__ __forceinline__ int32_t clamped(int32_t e) {
         return (int32_t)bfi(E::u, (uint32_t)e, (uint32_t)min(max(e, E::zero), E::hi));
     }
+    // the same, its bounds in registers
+    static __device__ __forceinline__ int32_t clamped3(int32_t e) {
+        return (int32_t)bfi(E::u, (uint32_t)e, (uint32_t)med3(e, E::zero, E::hi));
+    }
     // a sum after fast steps: only exact cancellation (+0) leaves it below zero
     static __device__ __forceinline__ int32_t settled(int32_t e) { return e < E::zero ? E::zero : clamped(e); }
-    // the step for any operands; a comes and goes clamped
-    __device__ __forceinline__ void xstep(int32_t &a, int32_t t, uint32_t r, int32_t &M) const {
-        t = clamped(t);
-        M = max(a, t);
+    // The step for any operands, in two parts, so that several chains' reads
+    // go out together; a comes and goes clamped
+    struct mid {
+        int32_t M, en;
+        uint32_t va;
+    };
+    __device__ __forceinline__ mid xread(int32_t a, int32_t t) const {
+        t = clamped3(t);
         const uint32_t va = at(a, t);
-        const int32_t x = sum(M, entry_any(va), draw(va, r));
-        a = !POS && va == tb + E::u ? E::zero : clamped(x);   // exact cancellation: +0
+        return {max(a, t), entry(va), va};
+    }
+    __device__ __forceinline__ int32_t xsum(const mid &m, uint32_t r) const {
+        const int32_t x = clamped3(sum(m.M, m.en, draw(m.va, r)));
+        return !POS && m.va == tb + E::u ? E::zero : x;   // exact cancellation: +0
     }
     // the xlns16 code of a sum
     static __device__ __forceinline__ uint32_t finish(int32_t e) {
@@ -1072,14 +1127,20 @@ __device__ __forceinline__ const char *e_image(const dev_tables &T) {
     if constexpr (MODE == LNSHIP_MONTE) return POS ? (const char *)T.emp : (const char *)T.em;
     else return POS ? (const char *)T.ebp : (const char *)T.eb;
 }
-// the table image into LDS, or (in_lds false) left in global memory
-template <int MODE, bool POS = false>
-__device__ __forceinline__ red_e<MODE, POS> stage_e(const dev_tables &T, char *lds, bool in_lds = true) {
+// The table image into LDS; TIGHT: base's narrow one, sb and db by distance
+template <int MODE, bool POS = false, bool TIGHT = false>
+__device__ __forceinline__ red_e<MODE, POS, TIGHT> stage_e(const dev_tables &T, char *lds) {
     using E = eform<MODE, POS>;
-    const char *img = e_image<MODE, POS>(T);
-    if (in_lds) stage_copy<8>(reinterpret_cast<int4 *>(lds), reinterpret_cast<const int4 *>(img), E::bytes / 16);
-    const uint32_t tb = in_lds ? lds_addr(lds) : 0u;
-    red_e<MODE, POS> R{tb, tb + E::cap, 1u << E::sh, in_lds ? nullptr : img};
+    const uint32_t tb = lds_addr(lds);
+    if constexpr (MODE == LNSHIP_BASE && TIGHT) {
+        typedef uint32_t __attribute__((address_space(3))) *lds_u32_t;
+        for (int i = threadIdx.x; i < k16_gauss_n; i += blockDim.x)
+            *(lds_u32_t)(uintptr_t)(tb + 4 * i) = (uint32_t)(uint16_t)T.gauss16[i] |
+                                                  (i == 0 ? 0x8000u : (uint32_t)(uint16_t)T.gauss16[k16_gauss_n + i]) << 16;
+    } else {
+        stage_copy<8>(reinterpret_cast<int4 *>(lds), reinterpret_cast<const int4 *>(e_image<MODE, POS>(T)), E::bytes / 16);
+    }
+    red_e<MODE, POS, TIGHT> R{tb, tb + E::cap, 1u << E::sh};
     asm("" : "+v"(R.tb), "+v"(R.cap), "+v"(R.scale));   // in registers (short encodings)
     return R;
 }
@@ -1223,9 +1284,6 @@ struct mm_args16 {
     // Monte start, monte_start(rms_seed, state, rms_offset)
     uint32_t rms_seed;
     uint64_t rms_offset;
-    // set by the launcher (base and Monte, one chain per lane): the rows leave
-    // no room for the adder's table in LDS
-    bool no_tab;
     uint32_t y0;   // set by the launcher: the column block of the grid's first row
     // set by the launcher: the grid is 2^xcd_sh times wider than the work;
     // workgroup x works (as block x >> xcd_sh) iff x is a multiple of 2^xcd_sh
@@ -1589,8 +1647,8 @@ __device__ __forceinline__ void mm16_chains(const mm_args16 &a, const dev_tables
 }
 
 // (defined with the other sequential row sums below)
-template <int MODE, bool POS>
-__device__ __forceinline__ uint32_t chain_e_pos(const red_e<MODE, POS> &R, uint32_t a, const uint16_t *row, int i0,
+template <int MODE, bool POS, bool TIGHT>
+__device__ __forceinline__ uint32_t chain_e_pos(const red_e<MODE, POS, TIGHT> &R, uint32_t a, const uint16_t *row, int i0,
                                                 int n, uint32_t st);
 template <class RED, bool POS = false>
 __device__ __forceinline__ void chain16(const RED &R, typename RED::acc_t &acc, const uint16_t *row, int i0, int n,
@@ -1602,9 +1660,9 @@ __device__ __forceinline__ void chain16(const RED &R, typename RED::acc_t &acc, 
 struct lfsr8_tab {
     uint32_t lo, t8;   // LDS byte addresses
 };
-__device__ __forceinline__ lfsr8_tab stage_lfsr8(const dev_tables &T, char *lds) {
-    stage_copy<2>(reinterpret_cast<int4 *>(lds), reinterpret_cast<const int4 *>(T.lfsr8), k_lfsr8_bytes / 16);
-    return {lds_addr(lds), lds_addr(lds) + 4096u};
+__device__ __forceinline__ lfsr8_tab stage_lfsr8(const dev_tables &T, char *lds, uint32_t at) {
+    stage_copy<2>(reinterpret_cast<int4 *>(lds + at), reinterpret_cast<const int4 *>(T.lfsr8), k_lfsr8_bytes / 16);
+    return {lds_addr(lds) + at, lds_addr(lds) + at + 4096u};
 }
 __device__ __forceinline__ i32x2 lfsr_draws8(const lfsr8_tab &L, uint32_t &s) {
     const uint32_t b = s & 255u, h = s >> 8;
@@ -1612,6 +1670,15 @@ __device__ __forceinline__ i32x2 lfsr_draws8(const lfsr8_tab &L, uint32_t &s) {
     s = h ^ (uint32_t) * (const uint16_t __attribute__((address_space(3))) *)(uintptr_t)(L.t8 + (b << 1));
     return x;
 }
+
+// Blocks that chains whose sums left the fast form's range run in the exact one
+// before they try the fast form again, so that failing costs at most a
+// sixteenth of the chains' time (several chains a lane, whose blocks are short
+// and whose exact form costs more: an eighth).
+constexpr int k_hold(int nc) { return nc == 1 ? 16 : 8; }
+// Whether the sums after an exact block are (in: a lane's are not) where the
+// fast form would fail: not for the few that a cancellation has left at zero
+__device__ __forceinline__ bool e_out(bool in) { return __popcll(__ballot(!in)) > 8; }
 
 // mm16_chains for base and Monte, over the one-word adders.  X32: the
 // activation rows are words in LDS ((log << sh) | u if negative), NC > 1; else
@@ -1706,41 +1773,50 @@ __device__ __forceinline__ void mme_chains(const mm_args16 &a, const dev_tables 
             for (int h = 0; h < 2; h++) {
                 const int u = 2 * i + h;
                 if (u < u0 || u >= u1) continue;
-                int32_t M[NC];
+                auto draw = [&](int j) {
+                    return monte ? __builtin_amdgcn_ubfe((uint32_t)(u < 4 ? dr[j].x : dr[j].y), 8 * (u & 3), 8) : 0u;
+                };
+                if constexpr (FAST) {
+                    int32_t M[NC];
 #pragma unroll
-                for (int j = 0; j < NC; j++) {
-                    uint32_t r = 0;
-                    if constexpr (monte) r = __builtin_amdgcn_ubfe((uint32_t)(u < 4 ? dr[j].x : dr[j].y), 8 * (u & 3), 8);
-                    if (u == 0 && start) {
-                        acc[j] = red_e<MODE>::clamped(t[j][h]);
-                        M[j] = E::hi;
-                    } else if constexpr (FAST) {
-                        R.step(acc[j], t[j][h], r, M[j]);
-                    } else {
-                        R.xstep(acc[j], t[j][h], r, M[j]);
+                    for (int j = 0; j < NC; j++) R.step(acc[j], t[j][h], draw(j), M[j]);
+#pragma unroll
+                    for (int j = 0; j < NC; j++) {
+                        mn = min(mn, M[j]);
+                        mx = max(mx, M[j]);
                     }
-                }
+                } else if (u == 0 && start) {
 #pragma unroll
-                for (int j = 0; j < NC; j++) {
-                    mn = min(mn, M[j]);
-                    mx = max(mx, M[j]);
+                    for (int j = 0; j < NC; j++) acc[j] = red_e<MODE>::clamped(t[j][h]);
+                } else {
+                    // (four chains at a time, Monte's eight two: more take
+                    // registers that cost a SIMD one or more of its waves)
+                    constexpr int B = monte && NC > 4 ? 2 : 4;
+#pragma unroll
+                    for (int j0 = 0; j0 < NC; j0 += B) {
+                        typename red_e<MODE>::mid md[B];
+#pragma unroll
+                        for (int j = j0; j < NC && j < j0 + B; j++) md[j - j0] = R.xread(acc[j], t[j][h]);
+#pragma unroll
+                        for (int j = j0; j < NC && j < j0 + B; j++) acc[j] = R.xsum(md[j - j0], draw(j));
+                        if (NC > B) __builtin_amdgcn_sched_barrier(0);
+                    }
                 }
             }
         }
     };
     // Group 0 (which starts the sums), then blocks of PF groups, then the
     // tail: blocks run in the fast form, and again in the exact one when a
-    // step left its range; the next block then starts exact, until one stays
-    // in range.  Group 0 and the tail run exact (one copy of each form's code).
-    // The next block's weights are loaded before a block runs.
-    bool exact = false;   // wave-uniform
+    // step left its range; the chains then stay exact for k_hold blocks, and
+    // until their sums are back in range.  Group 0 and the tail run exact.  The
+    // next block's weights are loaded before a block runs.
+    int hold = 0;   // exact blocks to come; wave-uniform, as exact
+    bool exact = false;
     const int groups = full + (tail > 0);
     uint4 wa[PF], wb[PF];
     mm16_wblock<PF>(a, m, zw, 1, wa);
     for (int g = 0, g1 = 1; g < groups; g = g1, g1 = min(g + PF, g < full ? full : groups)) {
         const bool body = g > 0 && g < full;
-        mn = E::hi;
-        mx = E::lo;
         bool redo = true;
         if (body) {
             mm16_wblock<PF>(a, m, zw, g + PF, wb);
@@ -1752,6 +1828,8 @@ __device__ __forceinline__ void mme_chains(const mm_args16 &a, const dev_tables 
                     a0[j] = acc[j];
                     s0[j] = st[j];
                 }
+                mn = E::hi;
+                mx = E::lo;
 #pragma unroll
                 for (int p = 0; p < PF; p++)
                     if (g + p < full) {
@@ -1767,25 +1845,36 @@ __device__ __forceinline__ void mme_chains(const mm_args16 &a, const dev_tables 
                         acc[j] = a0[j];
                         st[j] = s0[j];
                     }
-                    mn = E::hi;
-                    mx = E::lo;
+                    hold = k_hold(NC);
                 }
             }
-#pragma unroll
-            for (int p = 0; p < PF; p++) wa[p] = wb[p];
         }
         if (redo) {
+            bool in = true;
 #pragma unroll
             for (int j = 0; j < NC; j++) acc[j] = red_e<MODE>::settled(acc[j]);
-#pragma unroll 1
-            for (int q = g; q < g1; q++) {
-                grp_x xq[NC];
+            grp_x xq[NC];
+            if (body) {
 #pragma unroll
-                for (int j = 0; j < NC; j++) xq[j] = load_x(j, q);
-                group(std::false_type{}, load_w(q), xq, 0, q < full ? 8 : tail, q == 0);
+                for (int p = 0; p < PF; p++)
+                    if (g + p < full) {
+#pragma unroll
+                        for (int j = 0; j < NC; j++) xq[j] = load_x(j, g + p);
+                        group(std::false_type{}, wa[p], xq, 0, 8, false);
+                    }
+            } else {
+#pragma unroll
+                for (int j = 0; j < NC; j++) xq[j] = load_x(j, g);
+                group(std::false_type{}, load_w(g), xq, 0, g < full ? 8 : tail, g == 0);
             }
-            exact = __any(mn < E::lo || mx > E::hi) != 0;
+#pragma unroll
+            for (int j = 0; j < NC; j++) in = in && acc[j] >= E::lo && acc[j] <= E::hi;
+            hold = max(hold - 1, 0);
+            exact = hold > 0 || e_out(in);
         }
+        if (body)
+#pragma unroll
+            for (int p = 0; p < PF; p++) wa[p] = wb[p];
     }
 #pragma unroll
     for (int j = 0; j < NC; j++) res[j] = red_e<MODE>::finish(acc[j]) & 0xffffu;
@@ -1805,8 +1894,8 @@ __device__ __forceinline__ void mme_chains(const mm_args16 &a, const dev_tables 
 struct e_grp {
     uint4 q, s;   // codes; or logs and signs
 };
-template <int MODE, int PF, bool SPLIT, class B, class W, class X>
-__device__ __forceinline__ void chain_e(const red_e<MODE> &R, const lfsr8_tab &L8, int32_t &acc, uint32_t st, int k0,
+template <int MODE, int PF, bool SPLIT, bool TIGHT, class B, class W, class X>
+__device__ __forceinline__ void chain_e(const red_e<MODE, false, TIGHT> &R, const lfsr8_tab &L8, int32_t &acc, uint32_t st, int k0,
                                         int k1, const uint4 &w0, uint4 (&wa)[PF], B &&block, W &&load_w, X &&load_x) {
     using E = eform<MODE>;
     const int gf = k0 >> 3, full = k1 >> 3, tail = k1 & 7, groups = full + (tail > 0);
@@ -1816,18 +1905,19 @@ __device__ __forceinline__ void chain_e(const red_e<MODE> &R, const lfsr8_tab &L
         if constexpr (SPLIT) e_pair_split<MODE>(w, x, xs, km.lm, km.su, lm, sg);
         else e_pair<MODE>(w, x, km.lm, km.su, lm, sg);
     };
-    auto pair = [&](uint32_t w, uint32_t x, uint32_t xs, int32_t (&t)[2]) {
+    auto pair = [&](uint32_t w, uint32_t x, uint32_t xs, int32_t (&t)[2], bool clamp = false) {
         uint32_t lm, sg;
         half(w, x, xs, lm, sg);
+        if (clamp) lm = e_clamp(lm);
         e_words<MODE>(lm, sg, km.em, t);
     };
     // Monte's draws of a group, a byte each, and those of the next one, whose
     // table reads are in flight meanwhile
     i32x2 dr{0, 0}, drn{0, 0};
     auto draw_of = [&](int u) { return E::monte ? __builtin_amdgcn_ubfe((uint32_t)(u < 4 ? dr.x : dr.y), 8 * (u & 3), 8) : 0u; };
-    auto draws = [&](bool fast) __attribute__((always_inline)) {
+    auto draws = [&]() __attribute__((always_inline)) {
         if constexpr (E::monte) {
-            if (!fast && R.g) {   // no tables in LDS: step by step
+            if constexpr (TIGHT) {   // no tables of them: step by step
                 uint32_t d[2] = {0, 0};
 #pragma unroll
                 for (int u = 0; u < 8; u++) {
@@ -1844,12 +1934,16 @@ __device__ __forceinline__ void chain_e(const red_e<MODE> &R, const lfsr8_tab &L
     // first words of the next group, whose terms 0 and 1 it leaves there.  A
     // pair of products is formed in two parts, in the round trips of the two
     // steps before it, and the M of two steps recorded in that of a third.
+    // EX: the exact form, every product clamped, nothing recorded.
     int32_t t0 = 0, t1 = 0, Ma = E::hi, Mb = E::hi;
     auto note = [&] {
         asm("v_min3_i32 %0, %0, %1, %2" : "+v"(mn) : "v"(Ma), "v"(Mb));
         asm("v_max3_i32 %0, %0, %1, %2" : "+v"(mx) : "v"(Ma), "v"(Mb));
     };
-    auto fast8 = [&](const uint4 &wq, const e_grp &x, uint32_t wn, const e_grp &xn, int u0) __attribute__((always_inline)) {
+    auto pin = [&] { asm volatile("" ::"v"(mn), "v"(mx)); };   // note()'s work stays here
+    auto run8 = [&](auto ex_tag, const uint4 &wq, const e_grp &x, uint32_t wn, const e_grp &xn, int u0)
+                    __attribute__((always_inline)) {
+        constexpr bool EX = decltype(ex_tag)::value;
         const uint32_t ww[5] = {wq.x, wq.y, wq.z, wq.w, wn}, xx[5] = {x.q.x, x.q.y, x.q.z, x.q.w, xn.q.x};
         const uint32_t xs[5] = {x.s.x, x.s.y, x.s.z, x.s.w, xn.s.x};
 #pragma unroll
@@ -1858,17 +1952,30 @@ __device__ __forceinline__ void chain_e(const red_e<MODE> &R, const lfsr8_tab &L
             uint32_t lm = 0, sg = 0;
             auto even = [&] {
                 half(ww[i + 1], xx[i + 1], xs[i + 1], lm, sg);
-                note();
-                asm volatile("" ::"v"(mn), "v"(mx), "v"(lm), "v"(sg));
+                if constexpr (!EX) {
+                    note();
+                    pin();
+                }
+                asm volatile("" ::"v"(lm), "v"(sg));
             };
-            if (2 * i >= u0) M0 = R.step1(acc, t0, draw_of(2 * i), even);
-            else even();
-            if (i == 0) draws(true);
-            Mb = R.step1(acc, t1, draw_of(2 * i + 1), [&] {
+            auto odd = [&] {
+                if constexpr (EX) lm = e_clamp(lm);
                 e_words<MODE>(lm, sg, km.em, tn);
                 asm volatile("" ::"v"(tn[0]), "v"(tn[1]));
-            });
-            Ma = M0;
+            };
+            if (2 * i < u0) {
+                even();
+            } else {
+                if constexpr (EX) R.xstep1(acc, t0, draw_of(2 * i), even);
+                else M0 = R.step1(acc, t0, draw_of(2 * i), even);
+            }
+            if (i == 0) draws();
+            if constexpr (EX) {
+                R.xstep1(acc, t1, draw_of(2 * i + 1), odd);
+            } else {
+                Mb = R.step1(acc, t1, draw_of(2 * i + 1), odd);
+                Ma = M0;
+            }
             t0 = tn[0];
             t1 = tn[1];
         }
@@ -1878,84 +1985,93 @@ __device__ __forceinline__ void chain_e(const red_e<MODE> &R, const lfsr8_tab &L
     auto exact8 = [&](const uint4 &wq, const e_grp &x, int u0, int u1, bool start) __attribute__((always_inline)) {
         const uint32_t ww[4] = {wq.x, wq.y, wq.z, wq.w}, xx[4] = {x.q.x, x.q.y, x.q.z, x.q.w};
         const uint32_t xs[4] = {x.s.x, x.s.y, x.s.z, x.s.w};
-        draws(false);
+        draws();
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             if (u < u0 || u >= u1) continue;
-            int32_t t[2], M = E::hi;
+            int32_t t[2];
             pair(ww[u >> 1], xx[u >> 1], xs[u >> 1], t);
             if (u == 0 && start) acc = red_e<MODE>::clamped(t[0]);
-            else R.xstep(acc, t[u & 1], draw_of(u), M);
-            mn = min(mn, M);
-            mx = max(mx, M);
+            else acc = R.xsum(R.xread(acc, t[u & 1]), draw_of(u));
         }
         dr = drn;
     };
-    draws(false);
+    draws();
     dr = drn;
-    // as mme_chains: the first group, blocks of PF groups, the tail; a group
-    // or block that left the fast form's range runs again exactly, and so
-    // does the next block, until one stays in range.  The tail, and a first
-    // group that is not a whole one from term 0, run exactly.
-    bool exact = R.g != nullptr;
+    // As mme_chains: the first group, blocks of PF groups, the tail; a group
+    // or block that left the fast form's range runs again exactly (after the
+    // first group the next block too: its terms hold zeros).  The tail, and a
+    // first group that is not a whole one from term 0, run exactly.
+    int hold = 0;
+    bool exact = false;
     uint4 wb[PF];
     for (int g = gf, g1 = gf + 1; g < groups; g = g1, g1 = min(g + PF, g < full ? full : groups)) {
-        mn = E::hi;
-        mx = E::lo;
         bool redo = true;
-        if (g < full && (g > gf || k0 == 0)) {
+        const bool whole = g < full && (g > gf || k0 == 0);
+        if (g > gf && g < full) block(wb, g + PF);
+        if (whole && !exact) {
             const int32_t a0 = acc;
             const uint32_t s0 = st;
             const i32x2 d0 = dr;
-            if (g > gf) block(wb, g + PF);
-            if (!exact) {
-                int32_t t[2];
-                Ma = Mb = E::hi;
-                if (g == gf) {
-                    const e_grp x0 = load_x(gf);
-                    pair(w0.x, x0.q.x, x0.s.x, t);
-                    acc = red_e<MODE>::clamped(t[0]);
-                    t1 = t[1];
-                    fast8(w0, x0, w0.x, x0, 1);
-                } else {
-                    e_grp x[PF];
+            mn = Ma = Mb = E::hi;
+            mx = E::lo;
+            int32_t t[2];
+            if (g == gf) {
+                const e_grp x0 = load_x(gf);
+                pair(w0.x, x0.q.x, x0.s.x, t);
+                acc = red_e<MODE>::clamped(t[0]);
+                t1 = t[1];
+                run8(std::false_type{}, w0, x0, w0.x, x0, 1);
+            } else {
+                e_grp x[PF];
 #pragma unroll
-                    for (int p = 0; p < PF; p++) x[p] = load_x(g + p);
-                    pair(wa[0].x, x[0].q.x, x[0].s.x, t);
-                    t0 = t[0];
-                    t1 = t[1];
+                for (int p = 0; p < PF; p++) x[p] = load_x(g + p);
+                pair(wa[0].x, x[0].q.x, x[0].s.x, t);
+                t0 = t[0];
+                t1 = t[1];
 #pragma unroll
-                    for (int p = 0; p < PF; p++)
-                        if (g + p < full)
-                            fast8(wa[p], x[p], wa[p + 1 < PF ? p + 1 : p].x, x[p + 1 < PF ? p + 1 : p], 0);
-                }
-                note();
-                redo = __any(mn < E::lo || mx > E::hi) != 0;
-                if (redo) {
-                    acc = a0;
-                    st = s0;
-                    dr = d0;
-                    mn = E::hi;
-                    mx = E::lo;
-                }
+                for (int p = 0; p < PF; p++)
+                    if (g + p < full)
+                        run8(std::false_type{}, wa[p], x[p], wa[p + 1 < PF ? p + 1 : p].x, x[p + 1 < PF ? p + 1 : p], 0);
             }
-            if (g > gf)
-#pragma unroll
-                for (int p = 0; p < PF; p++) wa[p] = wb[p];
+            note();
+            redo = __any(mn < E::lo || mx > E::hi) != 0;
+            if (redo) {
+                acc = a0;
+                st = s0;
+                dr = d0;
+                hold = g > gf ? k_hold(1) : 2;
+            }
         }
-        if (redo) {
+        if (__builtin_expect(redo, 0)) {   // (out of the fast form's way in the instruction cache)
             acc = red_e<MODE>::settled(acc);
-#pragma unroll 1
-            for (int q = g; q < g1; q++)
-                exact8(load_w(q), load_x(q), q == gf ? k0 & 7 : 0, q < full ? 8 : tail, q == 0);
-            exact = R.g != nullptr || (g > gf && __any(mn < E::lo || mx > E::hi) != 0);
+            if (g > gf && g < full) {
+                e_grp x[PF];
+                int32_t t[2];
+#pragma unroll
+                for (int p = 0; p < PF; p++) x[p] = load_x(g + p);
+                pair(wa[0].x, x[0].q.x, x[0].s.x, t, true);
+                t0 = t[0];
+                t1 = t[1];
+#pragma unroll
+                for (int p = 0; p < PF; p++)
+                    if (g + p < full)
+                        run8(std::true_type{}, wa[p], x[p], wa[p + 1 < PF ? p + 1 : p].x, x[p + 1 < PF ? p + 1 : p], 0);
+            } else {
+                exact8(load_w(g), load_x(g), g == gf ? k0 & 7 : 0, g < full ? 8 : tail, g == 0);
+            }
+            hold = max(hold - 1, 0);
+            exact = hold > 0 || e_out(acc >= E::lo && acc <= E::hi);
         }
+        if (g > gf && g < full)
+#pragma unroll
+            for (int p = 0; p < PF; p++) wa[p] = wb[p];
     }
 }
 
 // mme_chains for one chain per lane; head: its first weights
-template <int MODE, int PF, bool XL, bool SPLIT, bool HEAD>
-__device__ __forceinline__ uint32_t mme_chain1(const mm_args16 &a, const dev_tables &T, const red_e<MODE> &R,
+template <int MODE, int PF, bool XL, bool SPLIT, bool HEAD, bool TIGHT>
+__device__ __forceinline__ uint32_t mme_chain1(const mm_args16 &a, const dev_tables &T, const red_e<MODE, false, TIGHT> &R,
                                                const lfsr8_tab &L8, const uint16_t *xl, int64_t m, int64_t z,
                                                int64_t zw, int64_t zx, int64_t n0, const mm_head<PF> &head) {
     const uint16_t *ws = a.w + zw * a.w_slice + m * 8;
@@ -1986,7 +2102,7 @@ __device__ __forceinline__ uint32_t mme_chain1(const mm_args16 &a, const dev_tab
         mm16_wblock<PF>(a, m, zw, 1, wa);
     }
     int32_t acc = eform<MODE>::zero;
-    chain_e<MODE, PF, SPLIT>(R, L8, acc, st, 0, (int)a.K, HEAD ? head.w0 : load_w(0), wa,
+    chain_e<MODE, PF, SPLIT, TIGHT>(R, L8, acc, st, 0, (int)a.K, HEAD ? head.w0 : load_w(0), wa,
                       [&](uint4 (&w)[PF], int g) { mm16_wblock<PF>(a, m, zw, g, w); }, load_w, load_x);
     return red_e<MODE>::finish(acc) & 0xffffu;
 }
@@ -2004,8 +2120,12 @@ __device__ __forceinline__ uint32_t mme_chain1(const mm_args16 &a, const dev_tab
 // logs and signs of chain_e's SPLIT.  RG groups of k_block rows share the rows
 // of several columns, so that long rows leave room for enough waves
 // RB: rows of a column group (k_block, or 64 for column groups of one wave)
-template <int MODE, int NC, int PF, bool XL, int CG, int W = 64, bool X32 = false, int RG = 1, int RB = k_block>
-__global__ __launch_bounds__(RB *CG *RG) void k_mm16(mm_args16 a, dev_tables T) {
+// TIGHT (base and Monte, one chain per lane): red_e
+// The waves a SIMD must hold: eight Monte chains a lane would take registers
+// that leave it two (K 64, M 1500, 2048 expert slots: 764 us at two, 653 at three)
+constexpr int mm16_waves(int mode, int nc, int rg) { return mode == LNSHIP_MONTE && nc == 8 && rg == 1 ? 3 : 1; }
+template <int MODE, int NC, int PF, bool XL, int CG, int W = 64, bool X32 = false, int RG = 1, int RB = k_block, bool TIGHT = false>
+__global__ __launch_bounds__(RB *CG *RG, mm16_waves(MODE, NC, RG)) void k_mm16(mm_args16 a, dev_tables T) {
     static_assert(!X32 || (is_e<MODE> && XL && CG == 1), "word rows: base and Monte");
     static_assert(RG == 1 || (X32 && NC > 1), "row groups share word rows");
     static_assert(RB == k_block || (W == 64 && RG == 1), "whole waves");
@@ -2036,14 +2156,14 @@ __global__ __launch_bounds__(RB *CG *RG) void k_mm16(mm_args16 a, dev_tables T) 
     mm_head<PF> hw{};
     if (head && live && a.K > 0) hw = mm16_head<PF>(a, m, zw);
     const auto R = [&] {
-        if constexpr (is_e<MODE>) return stage_e<MODE>(T, lds, !a.no_tab);
+        if constexpr (is_e<MODE>) return stage_e<MODE, false, TIGHT>(T, lds);
         else return stage_for<MODE, NC == 1>(T, lds);
     }();
     lfsr8_tab L8{};
-    if (MODE == LNSHIP_MONTE && !a.no_tab) L8 = stage_lfsr8(T, lds + eform<LNSHIP_MONTE>::bytes);
+    if (MODE == LNSHIP_MONTE && !TIGHT) L8 = stage_lfsr8(T, lds, eform<LNSHIP_MONTE>::bytes);
     constexpr int slot_bytes = MODE == LNSHIP_LPVIP ? lp_slot_bytes(NC) : 0;
     uint32_t *slots = reinterpret_cast<uint32_t *>(lds + mm16_tab_bytes<MODE>()) + (threadIdx.x >> 6) * (64 * NC);
-    uint16_t *xl = reinterpret_cast<uint16_t *>(lds + (is_e<MODE> && a.no_tab ? 0 : mm16_tab_bytes<MODE>() + slot_bytes));
+    uint16_t *xl = reinterpret_cast<uint16_t *>(lds + (TIGHT ? mm_xl_offset<MODE>() : mm16_tab_bytes<MODE>() + slot_bytes));
     // The RMS_NORM and MUL nodes before the product (norm): each workgroup
     // forms the scales of its own columns' rows, as k_rms16 does: the
     // squares into the activation rows' LDS, then one row's chain per lane
@@ -2482,12 +2602,12 @@ __device__ __forceinline__ void chain16(const RED &R, typename RED::acc_t &acc, 
 
 // chain16<RED, true> for base and Monte over the one-word adder: the xlns16
 // code of a (+) row[i0] (+) .. (+) row[n-1], every operand a positive code.
-// Blocks of four groups in the fast form, again in the exact one when one
-// left its range (as mme_chain1; positive sums only grow, so a block's ends
-// tell).  st: the LFSR state before the first draw.  POS: the positive
-// table, else the full one.
-template <int MODE, bool POS>
-__device__ __forceinline__ uint32_t chain_e_pos(const red_e<MODE, POS> &R, uint32_t a, const uint16_t *row, int i0,
+// Such sums only grow and every operand is in the log field, so only the upper
+// clamp is ever needed: blocks of four groups run without it, and again with
+// it when their sum passed the field.  st: the LFSR state before the first
+// draw.  POS: the positive table, else the full one.
+template <int MODE, bool POS, bool TIGHT>
+__device__ __forceinline__ uint32_t chain_e_pos(const red_e<MODE, POS, TIGHT> &R, uint32_t a, const uint16_t *row, int i0,
                                                 int n, uint32_t st) {
     using E = eform<MODE, POS>;
     constexpr int PF = 4;
@@ -2502,62 +2622,53 @@ __device__ __forceinline__ uint32_t chain_e_pos(const red_e<MODE, POS> &R, uint3
         if constexpr (E::monte) st = lfsr_step(st);
         return st >> 10;
     };
-    bool exact = false;
+    // terms u0 <= u < u1 of a group with the clamp
+    auto clamped8 = [&](const uint4 &v, int u0, int u1) __attribute__((always_inline)) {
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (u >= u0 && u < u1) {
+                const uint32_t r = next_draw();
+                R.step1(acc, word(w[u >> 1], u), r, [] {});
+                acc = min(acc, E::hi);
+            }
+    };
     uint4 cur[PF], nxt[PF];
+    const uint4 v0 = ld(g0), vl = ld(gl);
 #pragma unroll
     for (int p = 0; p < PF; p++) cur[p] = ld(g0 + 1 + p);
-    // the first group and the last run exact (with their bounds), the blocks
-    // between them fast
-    for (int g = g0, g1 = g0 + 1; g <= gl; g = g1, g1 = min(g + PF, g < gl ? gl : gl + 1)) {
-        bool redo = true;
-        if (g > g0 && g < gl) {
+    clamped8(v0, i0 & 7, min(n - 8 * g0, 8));
+    for (int g = g0 + 1; g < gl; g += PF) {
 #pragma unroll
-            for (int p = 0; p < PF; p++) nxt[p] = ld(g + PF + p);
-            if (!exact) {
-                const int32_t a0 = acc;
-                const uint32_t s0 = st;
-                int32_t t = word(cur[0].x, 0);
+        for (int p = 0; p < PF; p++) nxt[p] = ld(g + PF + p);
+        const int32_t a0 = acc;
+        const uint32_t s0 = st;
+        int32_t t = word(cur[0].x, 0);
 #pragma unroll
-                for (int p = 0; p < PF; p++) {
-                    if (g + p >= gl) break;
-                    const uint32_t w[5] = {cur[p].x, cur[p].y, cur[p].z, cur[p].w, cur[p + 1 < PF ? p + 1 : p].x};
+        for (int p = 0; p < PF; p++) {
+            if (g + p >= gl) break;
+            const uint32_t w[5] = {cur[p].x, cur[p].y, cur[p].z, cur[p].w, cur[p + 1 < PF ? p + 1 : p].x};
 #pragma unroll
-                    for (int u = 0; u < 8; u++) {
-                        int32_t tn;
-                        const uint32_t r = next_draw();
-                        R.step1(acc, t, r, [&] {
-                            tn = word(w[(u + 1) >> 1], u + 1);
-                            asm volatile("" ::"v"(tn));
-                        });
-                        t = tn;
-                    }
-                }
-                redo = __any(a0 < E::lo || acc > E::hi) != 0;
-                if (redo) {
-                    acc = a0;
-                    st = s0;
-                }
+            for (int u = 0; u < 8; u++) {
+                int32_t tn;
+                const uint32_t r = next_draw();
+                R.step1(acc, t, r, [&] {
+                    tn = word(w[(u + 1) >> 1], u + 1);
+                    asm volatile("" ::"v"(tn));
+                });
+                t = tn;
             }
-#pragma unroll
-            for (int p = 0; p < PF; p++) cur[p] = nxt[p];
         }
-        if (redo) {
+        if (__any(acc > E::hi)) {
+            acc = a0;
+            st = s0;
 #pragma unroll 1
-            for (int q = g; q < g1; q++) {
-                const uint4 v = ld(q);
-                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-                const int u0 = q == g0 ? i0 & 7 : 0, u1 = min(n - 8 * q, 8);
-#pragma unroll
-                for (int u = 0; u < 8; u++)
-                    if (u >= u0 && u < u1) {
-                        int32_t M;
-                        const uint32_t r = next_draw();
-                        R.xstep(acc, word(w[u >> 1], u), r, M);
-                    }
-            }
-            exact = R.g != nullptr || __any(acc < E::lo || acc > E::hi) != 0;
+            for (int q = g; q < min(g + PF, gl); q++) clamped8(ld(q), 0, 8);
         }
+#pragma unroll
+        for (int p = 0; p < PF; p++) cur[p] = nxt[p];
     }
+    if (gl > g0) clamped8(vl, 0, n - 8 * gl);
     return red_e<MODE, POS>::finish(acc) & 0xffffu;
 }
 
@@ -3572,7 +3683,7 @@ __device__ __forceinline__ uint32_t row_chain_e(const red_e<MODE> &R, const lfsr
     uint4 wa[PF];
     block(wa, (k0 >> 3) + 1);
     int32_t acc = e_of<MODE>(a);
-    chain_e<MODE, PF, false>(R, L8, acc, st, k0, k1, load_w(k0 >> 3), wa, block, load_w, load_x);
+    chain_e<MODE, PF, false, false>(R, L8, acc, st, k0, k1, load_w(k0 >> 3), wa, block, load_w, load_x);
     return red_e<MODE>::finish(acc) & 0xffffu;
 }
 
@@ -3651,7 +3762,7 @@ __global__ __launch_bounds__(k_block) void k_attn16(attn_args a, dev_tables T) {
         else return stage_for<MODE, true>(T, lds);
     }();
     lfsr8_tab L8{};
-    if constexpr (MODE == LNSHIP_MONTE) L8 = stage_lfsr8(T, lds + eform<MODE>::bytes);
+    if constexpr (MODE == LNSHIP_MONTE) L8 = stage_lfsr8(T, lds, eform<MODE>::bytes);
     const int hd = a.hd, n = a.n_kv, hp = (hd + 7) & ~7, rs = (n + 7) & ~7;
     uint16_t *xq = reinterpret_cast<uint16_t *>(lds + mm16_tab_bytes<MODE>());   // the query's codes
     uint16_t *c = xq + hp;                                                       // scores, then exps
@@ -4481,25 +4592,26 @@ static mm16_shape mm16_choose(int mode, int64_t M, int64_t N, int64_t nslices, i
     return {nc, 1, mm16_xl(mode, nc, kp), k_block};
 }
 
-template <int MODE, int NC, bool XL, int CG, int W = 64, bool X32 = false, int RG = 1, int RB = k_block>
+template <int MODE, int NC, bool XL, int CG, int W = 64, bool X32 = false, int RG = 1, int RB = k_block, bool TIGHT = false>
 static int launch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslices, int cus, hipStream_t st) {
     // prefetch depth within 128 VGPRs at four waves per SIMD
     constexpr int PF = NC == 1 ? (CG * RB >= 4 * k_block ? 4 : 8) : NC == 2 ? 2 : (NC == 4 && CG < 4) ? 2 : 1;
     const int rows_lds = (XL ? (int)(NC * CG * m.kp * (X32 ? 4 : 2)) + k_xl_pad : 0) + (MODE == LNSHIP_LPVIP ? lp_slot_bytes(NC) : 0);
-    const bool no_tab = is_e<MODE> && NC == 1 && !X32 && mm16_tab_bytes<MODE>() + rows_lds > k_lds_bytes - 1024;
-    const int lds = (no_tab ? 0 : mm16_tab_bytes<MODE>()) + rows_lds;
+    const int lds = (TIGHT ? mm_xl_offset<MODE>() : mm16_tab_bytes<MODE>()) + rows_lds;
+    if constexpr (is_e<MODE> && NC == 1 && XL && !X32 && !TIGHT)
+        if (lds > k_lds_bytes - 1024) return launch_mm16<MODE, 1, true, 1, W, false, 1, RB, true>(m, T, nslices, cus, st);
+    static_assert(!is_e<MODE> || MODE == LNSHIP_BASE || eform<MODE>::bytes <= mm_xl_offset<MODE>(), "Monte's table fits the narrow place");
     static_assert(PF * 16 <= k_xl_pad, "prefetch past the activation rows stays in the padding");
     // weight offsets within a block of PF groups are 32-bit
     if ((uint64_t)m.w_mstride * 16 * PF + (uint64_t)m.M * 16 > 0xffffffffu)
         return fail(LNSHIP_ERANGE, "mul_mat: weight rows too long for 32-bit block offsets%s");
     if (lds > 64 * 1024)
-        if (int rc = set_lds(k_mm16<MODE, NC, PF, XL, CG, W, X32, RG, RB>, lds)) return rc;
+        if (int rc = set_lds(k_mm16<MODE, NC, PF, XL, CG, W, X32, RG, RB, TIGHT>, lds)) return rc;
     constexpr int rows = W < 64 ? k_block / 64 * W : RB * RG;   // rows per workgroup
     dim3 grid((unsigned)((m.M + rows - 1) / rows), 1, (unsigned)nslices);
     if (grid.x > 2147483647u) return fail(LNSHIP_ERANGE, "mul_mat: grid too large%s");
     const int64_t blocks = (m.N + NC * CG - 1) / (NC * CG);   // of columns
     mm_args16 mx = m;
-    mx.no_tab = no_tab;
     mx.xcd_sh = MODE == LNSHIP_SUM32 ? xcd_shift((uint64_t)grid.x * (uint64_t)blocks * grid.z, cus) : 0;
     grid.x <<= mx.xcd_sh;
     // (more than one launch only where launch_mm16_x takes fewer columns a
@@ -4507,7 +4619,7 @@ static int launch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslices,
     for (int64_t y0 = 0; y0 < blocks; y0 += k_grid_y) {
         mx.y0 = (uint32_t)y0;
         grid.y = (unsigned)std::min(blocks - y0, k_grid_y);
-        hipLaunchKernelGGL((k_mm16<MODE, NC, PF, XL, CG, W, X32, RG, RB>), grid, dim3(RB * CG * RG), lds, st, mx, T);
+        hipLaunchKernelGGL((k_mm16<MODE, NC, PF, XL, CG, W, X32, RG, RB, TIGHT>), grid, dim3(RB * CG * RG), lds, st, mx, T);
         LNSHIP_HIP(hipGetLastError());
     }
     return 0;
