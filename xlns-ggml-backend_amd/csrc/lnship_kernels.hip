@@ -877,13 +877,13 @@ struct red16<LNSHIP_LPVIP> {
     __device__ __forceinline__ void add(acc_t &a, uint32_t v, uint32_t &st) const { add_ls(a, v & k16_logmask, v & k16_sign, st); }
     // add() of a positive v to a positive sum: sb only, the sign stays +
     __device__ __forceinline__ void add_pos(acc_t &a, uint32_t v, uint32_t &) const {
-        const uint32_t tl = (v & k16_logmask) << 16;
-        const uint32_t mx = max(a.l, tl), d = mx - min(a.l, tl);
-        const uint32_t u = ((0x1000000u - (d & 0x7fffffu)) >> 1) >> min(d >> 23, 31u);
-        const uint32_t pc = (uint32_t)(((uint64_t)u * (uint64_t)(0x800000u - u)) >> 23);
-        const int32_t adj = d < k32_esszer ? (int32_t)(u + (mul_u24(pc, 0x2B8u) >> 11)) : 0;
-        const uint32_t s = mx + (uint32_t)adj;
-        a.l = (s & k32_sign) ? ((s & k32_one) ? 0u : k32_logmask) : s;
+        // (front()'s steps for equal signs; the correction's last product fits
+        // 32 bits: u (2^23 - u) >> 23 < 2^21.  The sum only saturates.)
+        const uint32_t tl = (v & k16_logmask) << 16, mx = max(a.l, tl);
+        const uint32_t dq = min(sad_u32(a.l, tl, 0x800000u), k32_esszer + 0x800000u);
+        const uint32_t u = (0x1000000u - (dq & 0x7fffffu)) >> (dq >> 23), w = 0x800000u - u;
+        const uint32_t p = __builtin_amdgcn_alignbit(mulhi_u24(u, w), mul_u24(u, w), 23);
+        a.l = (uint32_t)__builtin_elementwise_add_sat((int32_t)mx, (int32_t)(u + (mul_u24(p, 0x2B8u) >> 11)));
     }
     __device__ __forceinline__ uint32_t finish(const acc_t &a) const { return (a.s | a.l) >> 16; }
 };
