@@ -448,6 +448,15 @@ int lnship_test_predict_skew(int skew);
  * previous value; host-side only, taking effect at the next launch.  No
  * counterpart in the reference. */
 int lnship_test_decode_width(int w);
+/* Test hook: the shape that lnship16_mul_mat (mode 0 to 3; with nslices =
+ * n_expert_used n_tokens and N = 1 lnship16_mul_mat_id) or lnship32_mul_mat
+ * (mode 4) launches on a device of cus CUs for K terms, M rows, N columns and
+ * nslices = ne12 ne13 activation slices.  shape receives eight values: columns
+ * a lane takes, column groups of a workgroup, rows of a group, whether the
+ * activation rows lie in LDS, rows of a wave, whether they take four bytes a
+ * value there, row groups that share them, whether the adder's tables are the
+ * narrow ones.  Host-side only.  No counterpart in the reference. */
+int lnship_test_mul_mat_shape(int mode, int64_t K, int64_t M, int64_t N, int64_t nslices, int cus, int *shape);
 
 /* Host: the (cos, sin) floats lns_rope uses for positions 0..n_pos-1 (the
  * float recurrence t *= powf(freq_base, -2/n_dims) per pair, cosf / sinf;

@@ -2123,7 +2123,7 @@ __device__ __forceinline__ uint32_t mme_chain1(const mm_args16 &a, const dev_tab
 // TIGHT (base and Monte, one chain per lane): red_e
 // The waves a SIMD must hold: eight Monte chains a lane would take registers
 // that leave it two (K 64, M 1500, 2048 expert slots: 764 us at two, 653 at three)
-constexpr int mm16_waves(int mode, int nc, int rg) { return mode == LNSHIP_MONTE && nc == 8 && rg == 1 ? 3 : 1; }
+constexpr int mm16_waves(int mode, int nc, int rg) { return mode == LNSHIP_MONTE && nc == 8 && rg == 1 ? 3 : 0; }   // (0: any)
 template <int MODE, int NC, int PF, bool XL, int CG, int W = 64, bool X32 = false, int RG = 1, int RB = k_block, bool TIGHT = false>
 __global__ __launch_bounds__(RB *CG *RG, mm16_waves(MODE, NC, RG)) void k_mm16(mm_args16 a, dev_tables T) {
     static_assert(!X32 || (is_e<MODE> && XL && CG == 1), "word rows: base and Monte");
@@ -4500,6 +4500,11 @@ struct mm16_shape {
     int nc, cg;   // columns per lane, column groups per workgroup
     bool xl;      // activations converted into LDS inside the kernel
     int rb;       // rows of a column group
+    int w;        // rows of a wave (64; single chains: fewer)
+    bool x32;     // (base, Monte) the rows in LDS at four bytes a value
+    int rg;       // row groups that share them
+    bool tight;   // red_e
+    int64_t most; // columns accepted: 65535 blocks of those first chosen
 };
 
 // The xlns32 tables leave room for one workgroup per CU, so the sum32 and
@@ -4517,8 +4522,8 @@ struct mm16_shape {
 static mm16_shape mm_shape_x32(int64_t M, int64_t N, int64_t nslices, int64_t kp, int cus, int max_nc) {
     // (one wave of several chains, or two waves of two or more, never wins)
     static const int shapes[][3] = {{1, 1, k_block}, {1, 2, k_block}, {1, 4, k_block}, {2, 4, k_block}, {4, 4, k_block},
-                                    {8, 4, k_block}, {1, 8, 64}, {1, 12, 64}, {1, 16, 64}, {2, 16, 64}, {4, 16, 64}};
-    mm16_shape best{1, 1, mm16_xl(LNSHIP_SUM32, 1, kp), k_block};
+                                    {8, 4, k_block}, {1, 8, 64}, {1, 12, 64}, {1, 16, 64}};
+    mm16_shape best{1, 1, mm16_xl(LNSHIP_SUM32, 1, kp), k_block, 64, false, 1, false, 0};
     int64_t best_cost = -1;
     for (const auto &sh : shapes) {
         const int nc = sh[0], cg = sh[1], rb = sh[2], waves = cg * rb / k_block;   // per SIMD
@@ -4538,7 +4543,10 @@ static mm16_shape mm_shape_x32(int64_t M, int64_t N, int64_t nslices, int64_t kp
         // ties go to more columns per workgroup (one weight decode serves
         // them), and to groups of k_block rows
         if (best_cost < 0 || (rb == 64 ? cost < best_cost : cost <= best_cost)) {
-            best = {nc, cg, xl, rb};
+            best.nc = nc;
+            best.cg = cg;
+            best.xl = xl;
+            best.rb = rb;
             best_cost = cost;
         }
     }
@@ -4586,10 +4594,61 @@ static uint32_t xcd_shift(uint64_t wgs, int cus) {
     return sh;
 }
 
+// The shape of a product's launch, from what the kernel stages.  The columns a
+// lane takes (mm16_nc) and whether the rows lie in LDS (mm16_xl) are chosen by
+// the tables and rows of codes that decide which calls are accepted.
+template <int MODE>
+static mm16_shape mm16_plan(int64_t M, int64_t N, int64_t nslices, int64_t kp, int cus) {
+    mm16_shape sh{};
+    if constexpr (MODE == LNSHIP_SUM32) {
+        sh = mm_shape_x32(M, N, nslices, kp, cus, 8);
+        if (sh.nc * sh.cg == 1 && sh.xl && narrow_mm(M * N * nslices, cus)) sh.w = 16;
+        sh.most = k_grid_y * sh.nc * sh.cg;
+        return sh;
+    }
+    sh.nc = mm16_nc(MODE, M, N, nslices, kp, cus);
+    sh.most = k_grid_y * sh.nc;
+    sh.cg = sh.rg = 1;
+    sh.xl = mm16_xl(MODE, sh.nc, kp);
+    sh.rb = k_block;
+    sh.w = 64;
+    if (!sh.xl) return sh;
+    auto lds = [&](int width) {
+        return mm16_tab_bytes<MODE>() + (MODE == LNSHIP_LPVIP ? lp_slot_bytes(sh.nc) : 0) + sh.nc * kp * width + k_xl_pad;
+    };
+    const int64_t room = k_lds_bytes - 1024;
+    // One column: the rows as logs and signs where they fit (per step: base 38
+    // ns either way, Monte 49 at code width, 46; K 1536, M 576, N 131: base
+    // 81.8 -> 75.1 us); several: as words
+    sh.x32 = is_e<MODE> && lds(4) <= room;
+    if (sh.nc == 1) {
+        if (const int w = narrow_w(MODE, M * N * nslices, cus)) sh.w = w;
+    } else if (sh.x32) {
+        // as many row groups as bring a CU to twelve waves, while the
+        // launch still has a workgroup for every CU (K 2048, M 8192, N
+        // 512, with one group: base 3692, Monte 1682 GMAC/s; with this
+        // rule 4220 and 2569)
+        const int64_t per_cu = k_lds_bytes / (lds(4) + 512), cols = (N + sh.nc - 1) / sh.nc * nslices;
+        while (sh.rg < 4 && per_cu * 4 * sh.rg < 12 && (M + 2 * sh.rg * k_block - 1) / (2 * sh.rg * k_block) * cols >= cus) sh.rg *= 2;
+    } else if (lds(2) > room) {
+        // Rows that fill the LDS beside what several chains take: one row per
+        // workgroup.  (Four rows, which would fit beside the tables of eight,
+        // leave a CU one workgroup of four waves: M 2048, N 512, Monte K 8192
+        // 6.28 ms against 3.40, base K 9704 4.61 against 2.88, lpvip K 9400
+        // 10.8 against 8.6.)
+        sh.nc = 1;
+    }
+    sh.tight = is_e<MODE> && !sh.x32 && lds(2) > room;
+    return sh;
+}
+
 static mm16_shape mm16_choose(int mode, int64_t M, int64_t N, int64_t nslices, int64_t kp, int cus) {
-    if (mode == LNSHIP_SUM32) return mm_shape_x32(M, N, nslices, kp, cus, 8);
-    const int nc = mm16_nc(mode, M, N, nslices, kp, cus);
-    return {nc, 1, mm16_xl(mode, nc, kp), k_block};
+    switch (mode) {
+        case LNSHIP_BASE: return mm16_plan<LNSHIP_BASE>(M, N, nslices, kp, cus);
+        case LNSHIP_MONTE: return mm16_plan<LNSHIP_MONTE>(M, N, nslices, kp, cus);
+        case LNSHIP_LPVIP: return mm16_plan<LNSHIP_LPVIP>(M, N, nslices, kp, cus);
+        default: return mm16_plan<LNSHIP_SUM32>(M, N, nslices, kp, cus);
+    }
 }
 
 template <int MODE, int NC, bool XL, int CG, int W = 64, bool X32 = false, int RG = 1, int RB = k_block, bool TIGHT = false>
@@ -4598,8 +4657,6 @@ static int launch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslices,
     constexpr int PF = NC == 1 ? (CG * RB >= 4 * k_block ? 4 : 8) : NC == 2 ? 2 : (NC == 4 && CG < 4) ? 2 : 1;
     const int rows_lds = (XL ? (int)(NC * CG * m.kp * (X32 ? 4 : 2)) + k_xl_pad : 0) + (MODE == LNSHIP_LPVIP ? lp_slot_bytes(NC) : 0);
     const int lds = (TIGHT ? mm_xl_offset<MODE>() : mm16_tab_bytes<MODE>()) + rows_lds;
-    if constexpr (is_e<MODE> && NC == 1 && XL && !X32 && !TIGHT)
-        if (lds > k_lds_bytes - 1024) return launch_mm16<MODE, 1, true, 1, W, false, 1, RB, true>(m, T, nslices, cus, st);
     static_assert(!is_e<MODE> || MODE == LNSHIP_BASE || eform<MODE>::bytes <= mm_xl_offset<MODE>(), "Monte's table fits the narrow place");
     static_assert(PF * 16 <= k_xl_pad, "prefetch past the activation rows stays in the padding");
     // weight offsets within a block of PF groups are 32-bit
@@ -4614,8 +4671,8 @@ static int launch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslices,
     mm_args16 mx = m;
     mx.xcd_sh = MODE == LNSHIP_SUM32 ? xcd_shift((uint64_t)grid.x * (uint64_t)blocks * grid.z, cus) : 0;
     grid.x <<= mx.xcd_sh;
-    // (more than one launch only where launch_mm16_x takes fewer columns a
-    // workgroup than the shape that dispatch_mm16 checked)
+    // (more than one launch only where mm16_plan takes fewer columns a
+    // workgroup than it chose first)
     for (int64_t y0 = 0; y0 < blocks; y0 += k_grid_y) {
         mx.y0 = (uint32_t)y0;
         grid.y = (unsigned)std::min(blocks - y0, k_grid_y);
@@ -4627,49 +4684,43 @@ static int launch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslices,
 
 template <int MODE, int NC, int CG, int RB = k_block>
 static int launch_mm16_x(const mm_args16 &m, const dev_tables &T, int64_t nslices, bool xl, int cus, hipStream_t st) {
-    if constexpr (is_e<MODE> && NC > 1) {
-        const int64_t lds = mm16_tab_bytes<MODE>() + (int64_t)NC * m.kp * 4 + k_xl_pad;
-        if (xl && lds <= k_lds_bytes - 1024) {
-            // as many row groups as bring a CU to twelve waves, while the
-            // launch still has a workgroup for every CU (K 2048, M 8192, N
-            // 512, with one group: base 3692, Monte 1682 GMAC/s; with this
-            // rule 4220 and 2569)
-            const int64_t per_cu = k_lds_bytes / (lds + 512), cols = (m.N + NC - 1) / NC * nslices;
-            int rg = 1;
-            while (rg < 4 && per_cu * 4 * rg < 12 && (m.M + 2 * rg * k_block - 1) / (2 * rg * k_block) * cols >= cus) rg *= 2;
-            switch (rg) {
-                case 4: return launch_mm16<MODE, NC, true, CG, 64, true, 4>(m, T, nslices, cus, st);
-                case 2: return launch_mm16<MODE, NC, true, CG, 64, true, 2>(m, T, nslices, cus, st);
-                default: return launch_mm16<MODE, NC, true, CG, 64, true>(m, T, nslices, cus, st);
-            }
-        }
-    }
-    if constexpr (NC > 1 && MODE != LNSHIP_SUM32) {
-        // Rows that fill the LDS beside what several chains take: one row per
-        // workgroup.  (Four rows, which would fit beside the tables of eight,
-        // leave a CU one workgroup of four waves: M 2048, N 512, Monte K 8192
-        // 6.28 ms against 3.40, base K 9704 4.61 against 2.88, lpvip K 9400
-        // 10.8 against 8.6.)
-        if (xl && mm16_tab_bytes<MODE>() + (MODE == LNSHIP_LPVIP ? lp_slot_bytes(NC) : 0) + (int64_t)NC * m.kp * 2 + k_xl_pad > k_lds_bytes - 1024)
-            return launch_mm16<MODE, 1, true, 1>(m, T, nslices, cus, st);
-    }
     return xl ? launch_mm16<MODE, NC, true, CG, 64, false, 1, RB>(m, T, nslices, cus, st)
               : launch_mm16<MODE, NC, false, CG, 64, false, 1, RB>(m, T, nslices, cus, st);
+}
+
+// base, Monte and lpvip: several columns a lane; one
+template <int MODE, int NC>
+static int launch_mm16_n(const mm_args16 &m, const dev_tables &T, int64_t nslices, const mm16_shape &sh, int cus,
+                         hipStream_t st) {
+    if constexpr (is_e<MODE>)
+        if (sh.x32) switch (sh.rg) {
+                case 4: return launch_mm16<MODE, NC, true, 1, 64, true, 4>(m, T, nslices, cus, st);
+                case 2: return launch_mm16<MODE, NC, true, 1, 64, true, 2>(m, T, nslices, cus, st);
+                default: return launch_mm16<MODE, NC, true, 1, 64, true>(m, T, nslices, cus, st);
+            }
+    return launch_mm16_x<MODE, NC, 1>(m, T, nslices, sh.xl, cus, st);
+}
+template <int MODE, int W>
+static int launch_mm16_1(const mm_args16 &m, const dev_tables &T, int64_t nslices, const mm16_shape &sh, int cus,
+                         hipStream_t st) {
+    if constexpr (is_e<MODE>) {
+        if (sh.x32) return launch_mm16<MODE, 1, true, 1, W, true>(m, T, nslices, cus, st);
+        if (sh.tight) return launch_mm16<MODE, 1, true, 1, W, false, 1, k_block, true>(m, T, nslices, cus, st);
+    }
+    return launch_mm16<MODE, 1, true, 1, W>(m, T, nslices, cus, st);
 }
 
 template <int MODE>
 static int dispatch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslices, const mm16_shape &sh,
                          int cus, hipStream_t st) {
-    if (m.N > k_grid_y * sh.nc * sh.cg) return fail(LNSHIP_ERANGE, "mul_mat: grid too large%s");
+    if (m.N > sh.most) return fail(LNSHIP_ERANGE, "mul_mat: grid too large%s");
     if constexpr (MODE == LNSHIP_SUM32) {
         // column groups: more waves per SIMD where the tables allow one
         // workgroup per CU
         if (sh.rb == 64) switch (sh.nc * 100 + sh.cg) {
                 case 108: return launch_mm16_x<MODE, 1, 8, 64>(m, T, nslices, sh.xl, cus, st);
                 case 112: return launch_mm16_x<MODE, 1, 12, 64>(m, T, nslices, sh.xl, cus, st);
-                case 116: return launch_mm16_x<MODE, 1, 16, 64>(m, T, nslices, sh.xl, cus, st);
-                case 216: return launch_mm16_x<MODE, 2, 16, 64>(m, T, nslices, sh.xl, cus, st);
-                default: return launch_mm16_x<MODE, 4, 16, 64>(m, T, nslices, sh.xl, cus, st);
+                default: return launch_mm16_x<MODE, 1, 16, 64>(m, T, nslices, sh.xl, cus, st);
             }
         switch (sh.nc * 10 + sh.cg) {
             case 12: return launch_mm16_x<MODE, 1, 2>(m, T, nslices, sh.xl, cus, st);
@@ -4678,38 +4729,21 @@ static int dispatch_mm16(const mm_args16 &m, const dev_tables &T, int64_t nslice
             case 44: return launch_mm16_x<MODE, 4, 4>(m, T, nslices, sh.xl, cus, st);
             case 84: return launch_mm16_x<MODE, 8, 4>(m, T, nslices, sh.xl, cus, st);
             default:
-                if (sh.xl && narrow_mm(m.M * m.N * nslices, cus))
-                    return launch_mm16<MODE, 1, true, 1, 16>(m, T, nslices, cus, st);
+                if (sh.w == 16) return launch_mm16<MODE, 1, true, 1, 16>(m, T, nslices, cus, st);
                 return launch_mm16_x<MODE, 1, 1>(m, T, nslices, sh.xl, cus, st);
         }
     } else {
-        switch (sh.nc) {
-            case 8: return launch_mm16_x<MODE, 8, 1>(m, T, nslices, sh.xl, cus, st);
-            case 4: return launch_mm16_x<MODE, 4, 1>(m, T, nslices, sh.xl, cus, st);
-            default:
-                if constexpr (is_e<MODE>) {
-                    // the rows as logs and signs where they fit (one column,
-                    // per step: base 38 ns either way, Monte 49 at code width,
-                    // 46; K 1536, M 576, N 131: base 81.8 -> 75.1 us)
-                    if (sh.xl && mm16_tab_bytes<MODE>() + m.kp * 4 + k_xl_pad <= k_lds_bytes - 1024)
-                        switch (narrow_w(MODE, m.M * m.N * nslices, cus)) {
-                            case 16: return launch_mm16<MODE, 1, true, 1, 16, true>(m, T, nslices, cus, st);
-                            case 32: return launch_mm16<MODE, 1, true, 1, 32, true>(m, T, nslices, cus, st);
-                            default: return launch_mm16<MODE, 1, true, 1, 64, true>(m, T, nslices, cus, st);
-                        }
-                }
-                if (sh.xl) switch (narrow_w(MODE, m.M * m.N * nslices, cus)) {
-                        case 4:
-                            if constexpr (MODE == LNSHIP_LPVIP) return launch_mm16<MODE, 1, true, 1, 4>(m, T, nslices, cus, st);
-                            break;
-                        case 8:
-                            if constexpr (MODE == LNSHIP_LPVIP) return launch_mm16<MODE, 1, true, 1, 8>(m, T, nslices, cus, st);
-                            break;
-                        case 16: return launch_mm16<MODE, 1, true, 1, 16>(m, T, nslices, cus, st);
-                        case 32: return launch_mm16<MODE, 1, true, 1, 32>(m, T, nslices, cus, st);
-                        default: break;
-                    }
-                return launch_mm16_x<MODE, 1, 1>(m, T, nslices, sh.xl, cus, st);
+        if (sh.nc == 8) return launch_mm16_n<MODE, 8>(m, T, nslices, sh, cus, st);
+        if (sh.nc == 4) return launch_mm16_n<MODE, 4>(m, T, nslices, sh, cus, st);
+        if (!sh.xl) return launch_mm16<MODE, 1, false, 1>(m, T, nslices, cus, st);
+        if constexpr (MODE == LNSHIP_LPVIP) {
+            if (sh.w == 4) return launch_mm16_1<MODE, 4>(m, T, nslices, sh, cus, st);
+            if (sh.w == 8) return launch_mm16_1<MODE, 8>(m, T, nslices, sh, cus, st);
+        }
+        switch (sh.w) {
+            case 16: return launch_mm16_1<MODE, 16>(m, T, nslices, sh, cus, st);
+            case 32: return launch_mm16_1<MODE, 32>(m, T, nslices, sh, cus, st);
+            default: return launch_mm16_1<MODE, 64>(m, T, nslices, sh, cus, st);
         }
     }
 }
@@ -5426,12 +5460,10 @@ static int mul_mat32_staged(device_state *s, const lnship_mul_mat_args *a, void 
                 wms, a->w_slice ? a->w_slice : kp * wms, dld, a->dst_slice ? a->dst_slice : a->N * dld};
     m.resid = a->residual;
     const mm16_shape sh = mm_shape_x32(m.M, m.N, nslices, kp, s->cus, 4);
-    if (sh.rb == 64) switch (sh.nc * 100 + sh.cg) {
-            case 108: return launch_mm32<1, 8, 64, false, 64>(m, s->T, nslices, s->cus, st);
-            case 112: return launch_mm32<1, 12, 64, false, 64>(m, s->T, nslices, s->cus, st);
-            case 116: return launch_mm32<1, 16, 64, false, 64>(m, s->T, nslices, s->cus, st);
-            case 216: return launch_mm32<2, 16, 64, false, 64>(m, s->T, nslices, s->cus, st);
-            default: return launch_mm32<4, 16, 64, false, 64>(m, s->T, nslices, s->cus, st);
+    if (sh.rb == 64) switch (sh.cg) {
+            case 8: return launch_mm32<1, 8, 64, false, 64>(m, s->T, nslices, s->cus, st);
+            case 12: return launch_mm32<1, 12, 64, false, 64>(m, s->T, nslices, s->cus, st);
+            default: return launch_mm32<1, 16, 64, false, 64>(m, s->T, nslices, s->cus, st);
         }
     switch (sh.nc * 10 + sh.cg) {
         case 12: return launch_mm32<1, 2>(m, s->T, nslices, s->cus, st);
@@ -5630,6 +5662,22 @@ int lnship16_rms_norm_mul(int mode, const float *src, const float *w, float *dst
 // k_attn16's soft_max total): lnship_test_predict_skew
 static uint32_t g_predict_skew = 0;
 
+int lnship_test_mul_mat_shape(int mode, int64_t K, int64_t M, int64_t N, int64_t nslices, int cus, int *shape) {
+    if (mode < 0 || mode > 4 || K < 0 || M < 1 || N < 1 || nslices < 1 || cus < 1 || !shape)
+        return fail(LNSHIP_EINVAL, "mul_mat_shape: bad argument%s");
+    const int64_t kp = (K + 7) & ~(int64_t)7;
+    mm16_shape sh;
+    if (mode == 4) {
+        sh = mm_shape_x32(M, N, nslices, kp, cus, 4);
+        sh.xl = sh.nc * sh.cg == 1 && kp > 0 && mm32_xl_fits(kp);
+        if (sh.nc * sh.cg == 1 && narrow_mm(M * N * nslices, cus)) sh.w = 16;
+    } else {
+        sh = mm16_choose(mode, M, N, nslices, kp, cus);
+    }
+    const int v[8] = {sh.nc, sh.cg, sh.rb, sh.xl, sh.w, sh.x32, sh.rg, sh.tight};
+    for (int i = 0; i < 8; i++) shape[i] = v[i];
+    return 0;
+}
 int lnship_test_decode_width(int w) {
     const int prev = g_decode_w;
     if (w == 0 || w == 16) g_decode_w = w;

@@ -153,6 +153,8 @@ def lib():
         "lnship32_add_lds": (ctypes.c_int, [ctypes.c_int, c_p, c_p, c_p, c_i64, c_p]),
         "lnship_test_predict_skew": (ctypes.c_int, [ctypes.c_int]),
         "lnship_test_decode_width": (ctypes.c_int, [ctypes.c_int]),
+        "lnship_test_mul_mat_shape": (ctypes.c_int, [ctypes.c_int, c_i64, c_i64, c_i64, c_i64, ctypes.c_int,
+                                                     ctypes.POINTER(ctypes.c_int)]),
         "lnship16_add": (ctypes.c_int, [c_p, c_p, c_i64, c_i64, c_p, c_p]),
         "lnship16_mul": (ctypes.c_int, [c_p, c_p, c_i64, c_i64, c_p, c_p]),
         "lnship16_swiglu": (ctypes.c_int, [c_p, c_i64, c_p, c_i64, c_p, c_i64, c_i64, c_p]),
