@@ -1321,8 +1321,8 @@ __device__ __forceinline__ uint32_t monte_start(const dev_tables &T, uint32_t se
 
 template <int MODE>
 constexpr int mm_xl_offset() { return (lds_tables_bytes<MODE>() + 15) & ~15; }
-// k_mm16's own tables: the one-word adders' for base and Monte, with the LFSR
-// tables when a lane runs several Monte chains
+// k_mm16's own tables: the one-word adders' for base and Monte, with Monte's
+// LFSR tables
 constexpr int k_lfsr8_bytes = 2 * 256 * 8 + 256 * 2;
 // (lpvip: lp_slots per wave beside the tables when a lane runs several chains)
 constexpr int lp_slot_bytes(int nc) { return nc > 1 ? k_block / 64 * 64 * nc * 4 : 0; }
@@ -1369,30 +1369,21 @@ __device__ __forceinline__ mm_head<PF> mm16_head(const mm_args16 &a, int64_t m, 
     return h;
 }
 
-// The K-long chains of lane m (output row m of slice z) over columns
+// sum32 and lpvip: the K-long chains of lane m (output row m) over columns
 // n0 .. n0 + nc: the weights from HBM, the activations from the LDS rows at
 // xl (XL) or the converted rows in scratch; each column's finished
 // accumulator (an xlns16 code) into res.  HEAD: the first weights come
 // loaded in head.
 template <int MODE, int NC, int PF, bool XL, bool HEAD = false>
-__device__ __forceinline__ void mm16_chains(const mm_args16 &a, const dev_tables &T, const red16<MODE> &R,
-                                            const uint16_t *xl, int64_t m, int64_t z, int64_t zw, int64_t zx,
-                                            int64_t n0, int nc, uint32_t (&res)[NC],
+__device__ __forceinline__ void mm16_chains(const mm_args16 &a, const red16<MODE> &R, const uint16_t *xl, int64_t m,
+                                            int64_t zw, int64_t zx, int64_t n0, int nc, uint32_t (&res)[NC],
                                             const mm_head<PF> &head = mm_head<PF>{}, uint32_t *slots = nullptr) {
     const int kp = (int)a.kp;
     const uint16_t *ws = a.w + zw * a.w_slice + m * 8;
     const uint16_t *xs = a.x + (zx * a.N + n0) * a.kp;
     const int64_t wstride = a.w_mstride * 8;   // between consecutive groups of 8 k
     typename red16<MODE>::acc_t acc[NC]{};
-    uint32_t st[NC];
-#pragma unroll
-    for (int j = 0; j < NC; j++) {
-        st[j] = 0;
-        if (MODE == LNSHIP_MONTE && j < nc) {
-            const uint64_t out = ((uint64_t)z * (uint64_t)a.M + (uint64_t)m) * (uint64_t)a.N + (uint64_t)(n0 + j);
-            st[j] = lfsr_jump(T, monte_start(T, a.seed, a.state, a.offset), out * (uint64_t)(a.K - 1));
-        }
-    }
+    uint32_t st = 0;   // (the adders' LFSR state: none here)
     const int K = (int)a.K;
     const int full = K >> 3, tail = K & 7;
     // Prefetches past the last group reload the last group: every load is
@@ -1539,8 +1530,8 @@ __device__ __forceinline__ void mm16_chains(const mm_args16 &a, const dev_tables
                 if (u >= u0 && u < u1) {
                     const uint32_t tl = (u & 1) ? pl[u >> 1] >> 16 : pl[u >> 1] & 0xffffu;
                     const uint32_t ts = ((u & 1) ? ps[u >> 1] >> 16 : ps[u >> 1]) & k16_sign;
-                    if (u == 0 && u0 < 0) acc[0] = R.start(ts | tl, st[0]);
-                    else R.add_ls(acc[0], tl, ts, st[0]);
+                    if (u == 0 && u0 < 0) acc[0] = R.start(ts | tl, st);
+                    else R.add_ls(acc[0], tl, ts, st);
                 }
             }
             return;
@@ -2132,8 +2123,8 @@ __global__ __launch_bounds__(RB *CG *RG, mm16_waves(MODE, NC, RG)) void k_mm16(m
     extern __shared__ __align__(16) char lds[];
     // a widened launch: the workgroups between the working ones leave at once
     if (blockIdx.x & ((1u << a.xcd_sh) - 1u)) return;
-    // CG column groups of k_block lanes each share the staged tables: group
-    // c takes columns [nw + c NC, nw + (c + 1) NC) of the same k_block rows
+    // CG column groups of RB lanes each share the staged tables: group c
+    // takes columns [nw + c NC, nw + (c + 1) NC) of the same RB rows
     const int cg = CG == 1 ? 0 : (int)(threadIdx.x / RB);
     const int64_t nw = ((int64_t)blockIdx.y + a.y0) * (NC * CG);
     const int64_t n0 = nw + (int64_t)cg * NC;
@@ -2145,7 +2136,7 @@ __global__ __launch_bounds__(RB *CG *RG, mm16_waves(MODE, NC, RG)) void k_mm16(m
     int64_t zw, zx;
     const bool slice_ok = mm_slices(a, z, i12, i13, zw, zx);
     const int lane = (int)(threadIdx.x & 63u);
-        constexpr bool dup = W < 64 && MODE != LNSHIP_SUM32;   // a chain on 64 / W lanes
+    constexpr bool dup = W < 64 && MODE != LNSHIP_SUM32;   // a chain on 64 / W lanes
     const int wr = dup ? lane / (64 / W) : lane;              // the lane's row in the wave
     const int64_t m = W < 64 ? (int64_t)(blockIdx.x >> a.xcd_sh) * (k_block / 64 * W) + (threadIdx.x >> 6) * W + wr
                              : (int64_t)(blockIdx.x >> a.xcd_sh) * (RB * RG) + (threadIdx.x % (RB * RG));
@@ -2300,7 +2291,7 @@ __global__ __launch_bounds__(RB *CG *RG, mm16_waves(MODE, NC, RG)) void k_mm16(m
     uint32_t res[NC];
     if constexpr (is_e<MODE> && NC == 1) res[0] = mme_chain1<MODE, PF, XL, X32, head>(a, T, R, L8, xl, m, z, zw, zx, n0, hw);
     else if constexpr (is_e<MODE>) mme_chains<MODE, NC, PF, XL, X32>(a, T, R, L8, xl, m, z, zw, zx, n0, nc, res);
-    else mm16_chains<MODE, NC, PF, XL, head>(a, T, R, xl, m, z, zw, zx, n0, nc, res, hw, slots);
+    else mm16_chains<MODE, NC, PF, XL, head>(a, R, xl, m, zw, zx, n0, nc, res, hw, slots);
     if (dup && lane % (64 / W) != 0) return;   // one lane of a chain stores
 #pragma unroll
     for (int j = 0; j < NC; j++)
@@ -2991,7 +2982,7 @@ __global__ __launch_bounds__(k_block) void k_mm16_rms(mm_args16 a, dev_tables T)
     // scale differs (every thread reads the same two words after the barrier)
     for (int pass = 0;; pass++) {
         if (active) {
-            mm16_chains<LNSHIP_SUM32, 1, PF, true, true>(a, T, R, xl, m, 0, 0, 0, 0, 1, res, hw);
+            mm16_chains<LNSHIP_SUM32, 1, PF, true, true>(a, R, xl, m, 0, 0, 0, 1, res, hw);
         } else if (pass == 0 && threadIdx.x == k_rms_mm_rows) {
             uint32_t st = 0;
             typename red16<LNSHIP_SUM32>::acc_t acc = R.start(0u, st);
@@ -4514,10 +4505,11 @@ struct mm16_shape {
 // 9 slices 138 us in groups of 256, 51 us in groups of 64; 576 x 576 by
 // 201 columns 160 -> 94 us).  Time per k of a
 // shape is rounds x (chains per SIMD) x (time per chain step at that many
-// waves per SIMD); measured on MI355X, a chain step costs 166 ns with one
-// wave and one chain (the adder's latency), 148 ns with one wave of several
-// chains, 103 ns at two waves, 91 at three and 85 ns at four (the VALU issue
-// rate of 49 instructions).
+// waves per SIMD), the last for an adder of 49 instructions, 166 ns with one
+// wave (its latency), 103 at two, 91 at three and 85 ns at four.  The present
+// one takes 112, 74, 67 and 65.5 ns (sum32, M 64 to 256, K 448 less K 208 over
+// full rounds; xlns32 106, 75, 73 and 66 to 71): the order of the shapes is the
+// same, the gain from more waves less than the rule counts.
 // max_nc: 8 (sum32, whose launches may stage their rows in LDS) or 4 (xlns32)
 static mm16_shape mm_shape_x32(int64_t M, int64_t N, int64_t nslices, int64_t kp, int cus, int max_nc) {
     // (one wave of several chains, or two waves of two or more, never wins)
@@ -4538,7 +4530,7 @@ static mm16_shape mm_shape_x32(int64_t M, int64_t N, int64_t nslices, int64_t kp
         if (rb == 64 && (wg_n > k_grid_y || wg_m * cg * rb > 0xffffffff)) continue;
         const int64_t wgs = wg_m * wg_n * nslices;
         const int64_t rounds = (wgs + std::max(cus, 1) - 1) / std::max(cus, 1);
-        const int64_t step = waves == 1 ? (nc == 1 ? 166 : 148) : waves == 2 ? 103 : waves == 3 ? 91 : 85;
+        const int64_t step = waves == 1 ? 166 : waves == 2 ? 103 : waves == 3 ? 91 : 85;
         const int64_t cost = rounds * waves * nc * step;
         // ties go to more columns per workgroup (one weight decode serves
         // them), and to groups of k_block rows
@@ -5153,7 +5145,7 @@ int lnship_init(void) {
     {
         // the one-word adders' tables (eform): sb(d) in slot 4 d, db(d) in the
         // slots beside it, exact cancellation in slot 1 (an adjustment that
-        // leaves any sum below zero).  Monte: see red_e::adjusted
+        // leaves any sum below zero).  Monte: red_e::sum
         std::vector<int16_t> eb(eform<LNSHIP_BASE>::bytes / 2, 0);
         std::vector<int32_t> em(eform<LNSHIP_MONTE>::bytes / 4, 0);
         for (int d = 0; d <= eform<LNSHIP_BASE>::far; d++) {
