@@ -2621,7 +2621,7 @@ __device__ __forceinline__ uint32_t chain_e_pos(const red_e<MODE, POS, TIGHT> &R
             if (u >= u0 && u < u1) {
                 const uint32_t r = next_draw();
                 R.step1(acc, word(w[u >> 1], u), r, [] {});
-                acc = min(acc, E::hi);
+                acc = min(acc, E::hi - (int32_t)E::u);   // (the sign stays +)
             }
     };
     uint4 cur[PF], nxt[PF];
