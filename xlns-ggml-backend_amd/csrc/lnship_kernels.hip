@@ -4866,6 +4866,7 @@ static int launch_sm16(sm_args &m, int64_t nrows, const dev_tables &T, int cus, 
     const int64_t waves = std::max<int64_t>(4, std::min<int64_t>(most, (((int64_t)m.rb << m.gs) + 63) / 64));
     // (a launch takes fewer than 2^32 threads)
     const int threads = (int)(wgs * waves < (int64_t)1 << 26 ? waves * 64 : k_block);
+    while (1 << m.gs > threads) m.gs--;
     const int lds = tab + (int)(m.rb * rs * 2);
     const dim3 grid((unsigned)wgs);
     auto go = [&](auto kernel) {
