@@ -1,6 +1,6 @@
 """lpvip products of several chains per lane against the oracle: additions whose
-exact branch few, most or all lanes need at once, zeros, ends of groups, every
-number of chains, rows that fill the LDS."""
+exact branch few, most or all lanes need at once, zeros, ends of groups, one and
+four chains a lane, rows that fill the LDS (one chain) or lie in scratch (eight)."""
 import numpy as np
 import pytest
 

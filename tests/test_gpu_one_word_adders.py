@@ -1,7 +1,7 @@
 """The base and Monte products and row sums against the oracle, bit for bit, where
 their block-wise fast form can go wrong: ends of groups and blocks, operands that
 leave the fast form's range (zeros, cancellation, underflow, overflow) at any
-place of a chain, every workgroup shape, rows that leave the adder's table no
+place of a chain, several workgroup shapes, rows that leave Monte's tables no
 room in LDS."""
 import numpy as np
 import pytest
@@ -76,13 +76,13 @@ def test_products(ln, mode, kind, K, M, N):
 
 
 @pytest.mark.parametrize("mode", MODES)
-@pytest.mark.parametrize("K,M,N", [(2048, 2048, 512),    # four row groups share long word rows
-                                   (1200, 1030, 530),    # two, ragged
+@pytest.mark.parametrize("K,M,N", [(2048, 2048, 512),    # two row groups share long word rows
+                                   (1200, 1030, 530),    # four columns a lane, ragged rows
                                    (5000, 300, 2100),    # word rows do not fit: code rows
-                                   (9704, 260, 2100),    # nor do eight code rows beside the table
+                                   (9704, 260, 2100),    # base: nor do eight code rows (one column); Monte: in scratch
                                    (30011, 40, 1),       # one column as logs and signs
                                    (40007, 40, 1),       # as codes: too long for both
-                                   (66000, 3, 1)])       # no room for the table (exact steps only)
+                                   (66000, 3, 1)])       # Monte: no room for all the tables
 def test_workgroup_shapes(ln, mode, K, M, N):
     print(f"\n[shapes] {mode} K={K} M={M} N={N}", flush=True)
     w, x = operands("plain", K, M, N, 5)

@@ -276,21 +276,22 @@ def _sample(n, step):
     return np.unique(np.concatenate([np.arange(0, n, step), [n - 1]]))
 
 
-# Shapes that select each workgroup shape of the xlns32-accumulating GEMVs on
-# a 256-CU MI355X: (columns per lane, column groups), and whether the
-# activations fit in LDS next to the tables.  Each output depends on its own
+# Shapes over the workgroup shapes of the xlns32-accumulating GEMVs on a
+# 256-CU MI355X: (columns per lane, column groups of 256 rows, or of 64), and
+# whether the activations fit in LDS next to the tables (sum32; xlns32's lie
+# in scratch but for one column).  Each output depends on its own
 # row and column only, so the big shapes are checked exactly on a sample of
 # rows x columns (every column group and wave slot is hit).
 X32_SHAPES = [
     # K,    M,    N      lane cols x groups
     (21, 64, 1),      # 1 x 1
     (21, 64, 384),    # 1 x 2
-    (21, 70, 768),    # 1 x 4, ragged rows
-    (21, 64, 2000),   # 2 x 4, ragged columns
-    (21, 300, 2048),  # 4 x 4
+    (21, 70, 768),    # 1 x 8 of 64, ragged rows
+    (21, 64, 2000),   # 1 x 8 of 64, ragged columns
+    (21, 300, 2048),  # 1 x 16 of 64
     (21, 1024, 2048),  # 8 x 4, activations in LDS
     (1000, 1024, 2048),  # 8 x 4, activations from global memory
-    (1701, 300, 2040),  # 4 x 4, activations from global memory, K tail
+    (1701, 300, 2040),  # 1 x 8 of 64, activations in LDS, K tail
 ]
 
 

@@ -1,7 +1,8 @@
 """sum32 and xlns32 products whose launches take column groups of one wave's rows
-(few rows, or rows that a 256-row group covers badly), against the oracle: rows
-and columns off the tiles, broadcast weight slices, K off the group of eight, a
-residual, activation rows in LDS and in scratch."""
+(few rows, or rows that a 256-row group covers badly), and three that stay with
+256-row groups beside them, against the oracle: rows and columns off the tiles,
+broadcast weight slices, K off the group of eight, activation rows in LDS (sum32)
+and in scratch (xlns32)."""
 import numpy as np
 import pytest
 
